@@ -113,7 +113,8 @@ int SNEPPX_qlinear_w8_gemv(const float* x, const int8_t* qweight, const float* s
 /* C2/C3/C5: W4A16.  x bf16 [M][K]; y [M][N] in y_dtype (SNEPPX_BFLOAT16 or
  * SNEPPX_FLOAT32); fp32 accumulation.  qzeros NULL => symmetric zero 8.
  * g_idx NULL => contiguous groups of `group` columns; otherwise g_idx[k] in
- * [0, G).  Small M runs the decode GEMV; large M the MFMA prefill GEMM. */
+ * [0, G).  Small M runs the decode GEMVs, a decode batch the batch kernel,
+ * large M the MFMA prefill GEMM. */
 int SNEPPX_qlinear_w4a16(const uint16_t* x, const uint32_t* qweight, const uint16_t* scales,
                          const uint32_t* qzeros, const int32_t* g_idx, size_t G,
                          const float* bias, void* y, SNEPPXDtype y_dtype, size_t M, size_t N,
@@ -180,9 +181,9 @@ int SNEPPX_qlinear_silu_mul(const uint16_t* gate_up, uint16_t* out, size_t T, si
  * projection [2F][K] in the W4 layout, gate rows first; bias is fp32 [2F]
  * or NULL.  out bf16 [M][F] = bf16(silu(g) * u) with g = x . Wg^T + bias[n]
  * and u = x . Wu^T + bias[F + n] kept in fp32 (no bf16 round trip of the
- * [M][2F] projection).  M >= 256 runs the prefill GEMM with the SwiGLU in
- * its epilogue; fewer rows run the decode linear into fp32 scratch, then
- * the same rule.  The exponential and reciprocal use the hardware's fast
+ * [M][2F] projection).  The prefill GEMM (large M), the batch kernel and the
+ * M = 1 kernel apply the SwiGLU in their epilogues; other shapes run the
+ * decode linear into fp32 scratch, then the same rule.  The exponential and reciprocal use the hardware's fast
  * approximations (about 1 ulp, below the bf16 rounding).  F % 8 == 0. */
 int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
                                 const uint16_t* scales, const uint32_t* qzeros, const float* bias,

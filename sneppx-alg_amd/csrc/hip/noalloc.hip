@@ -6,7 +6,7 @@
 // In host code the array's name is a host-side stand-in, not a device
 // address.  Its address on a device comes from hipGetSymbolAddress, looked up
 // once per device (with that device current, at the entry point's first call
-// there) and kept in g_scratch[dev]; only that pointer is ever handed to
+// there) and kept in known[dev]; only that pointer is ever handed to
 // kernels.  Each device has its own copy at its own address.
 #include <hip/hip_runtime.h>
 
@@ -20,15 +20,19 @@
 
 static __device__ __align__(256) uint8_t scratch[SNEPPX_NOALLOC_SCRATCH_BYTES];
 
-namespace {
-std::atomic<void*> g_scratch[snx::kMaxDevices];
-std::mutex g_scratch_mu;
-}  // namespace
+// Arrival counters of the K spans (zero when the library loads; every call
+// leaves them zero), apart from the scratch so that no other call writes them.
+constexpr size_t kCounterBytes = 64 << 10;
+static __device__ __align__(256) uint32_t counters[kCounterBytes / sizeof(uint32_t)];
 
-extern "C" void* snx_noalloc_scratch(size_t bytes, const char* who) {
-    if (bytes > (size_t)SNEPPX_NOALLOC_SCRATCH_BYTES) {
+namespace {
+std::atomic<void*> g_scratch[snx::kMaxDevices], g_counters[snx::kMaxDevices];
+std::mutex g_scratch_mu;
+
+void* static_array(const void* symbol, std::atomic<void*>* known, size_t bytes, size_t most, const char* who) {
+    if (bytes > most) {
         snx_set_error("%s: this call needs %zu bytes of scratch, more than the %zu of the "
-                      "library's static buffer", who, bytes, (size_t)SNEPPX_NOALLOC_SCRATCH_BYTES);
+                      "library's static buffer", who, bytes, most);
         return nullptr;
     }
     const int dev = snx::current_device();
@@ -36,18 +40,31 @@ extern "C" void* snx_noalloc_scratch(size_t bytes, const char* who) {
         snx_set_error("%s: no current device (or device index beyond %d)", who, snx::kMaxDevices - 1);
         return nullptr;
     }
-    void* p = g_scratch[dev].load(std::memory_order_acquire);
+    void* p = known[dev].load(std::memory_order_acquire);
     if (p) return p;
     std::lock_guard<std::mutex> lock(g_scratch_mu);
-    p = g_scratch[dev].load(std::memory_order_relaxed);
+    p = known[dev].load(std::memory_order_relaxed);
     if (!p) {
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+        const hipError_t e = hipGetSymbolAddress(&p, symbol);
         if (e != hipSuccess || !p) {
-            snx_set_error("%s: hipGetSymbolAddress(scratch) on device %d: %s", who, dev,
+            snx_set_error("%s: hipGetSymbolAddress on device %d: %s", who, dev,
                           hipGetErrorString(e));
             return nullptr;
         }
-        g_scratch[dev].store(p, std::memory_order_release);
+        known[dev].store(p, std::memory_order_release);
     }
     return p;
 }
+}  // namespace
+
+extern "C" {
+
+void* snx_noalloc_scratch(size_t bytes, const char* who) {
+    return static_array(HIP_SYMBOL(scratch), g_scratch, bytes, SNEPPX_NOALLOC_SCRATCH_BYTES, who);
+}
+
+void* snx_noalloc_counters(size_t bytes, const char* who) {
+    return static_array(HIP_SYMBOL(counters), g_counters, bytes, kCounterBytes, who);
+}
+
+}  // extern "C"

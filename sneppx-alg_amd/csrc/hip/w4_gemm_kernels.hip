@@ -811,6 +811,16 @@ int snx_w4a16_gemm_splits(size_t M, size_t N, size_t K) {
     return 1;
 }
 
+// Estimated time in units of 0.1 us, to set against the batch kernel's: the
+// activation pass and the kernel's fixed parts (16 us), and 1.6 us a step for
+// every round of the CUs.  splits: the K spans the call runs.
+size_t snx_w4a16_gemm_cost(size_t M, size_t N, size_t K, int splits) {
+    const size_t ntiles = ((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN);
+    const size_t ncu = (size_t)snx::cu_count(), nk = K / GBK;
+    const size_t full = ntiles / ncu, rem = ntiles % ncu;
+    return 160 + 16 * (full * nk + (rem ? nk / (size_t)splits : 0));
+}
+
 // Bytes of the span partials (`part`) and arrival counters (`cnt`) of a
 // `splits`-span call: a 16 KB slot per (unit, wave) of the tiles that take
 // spans (past a full round of CUs only the remaining ones), a counter per

@@ -10,8 +10,12 @@
 #include "snx_hip.h"
 #include "../snx_internal.h"
 
-/* rows from which W4A16 runs the MFMA GEMM instead of 64-row GEMV slices */
+/* rows from which W4A16 may run the prefill GEMM with an fp32 result: its
+ * fp32 sums are 2e-6 off where the batch kernel's are 1e-7 and those of the
+ * GEMVs before it 1e-6.  A bf16 result hides either; it may run the GEMM
+ * from half a row tile on. */
 #define SNX_W4_GEMM_MIN_M 256
+#define SNX_W4_GEMM_MIN_M_BF16 64
 
 static int aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
@@ -123,6 +127,57 @@ static void* w4_scratch(size_t bytes, int noalloc, SNEPPXStream stream) {
                    : snx_workspace(bytes, 1, stream);
 }
 
+/* The batch kernel with its scratch; glu: N gate/up pairs (see snx_k_w4a16_batch). */
+static int w4_batch(const char* who, int noalloc, const uint16_t* x, const uint32_t* qweight, const uint16_t* scales,
+                    const uint32_t* qzeros, const float* bias, void* y, int y_f32, size_t M, size_t N, size_t K,
+                    int group, int glu, SNEPPXStream stream) {
+    const size_t rows = glu ? 2 * N : N;
+    const int splits = snx_w4a16_batch_splits(M, rows, K);
+    void* part = NULL;
+    uint32_t* cnt = NULL;
+    if (splits > 1) {
+        const size_t pb = snx_w4a16_batch_part_bytes(M, rows, splits), cb = snx_w4a16_batch_cnt_bytes(M, rows);
+        part = noalloc ? snx_noalloc_scratch(pb, who) : snx_workspace(pb, 3, stream);
+        cnt = (uint32_t*)(noalloc ? snx_noalloc_counters(cb, who) : snx_workspace_zeroed(cb, 4, stream));
+        if (!part || !cnt) return -1;
+    }
+    return snx_k_w4a16_batch(x, qweight, scales, qzeros, y, bias, y_f32, M, N, K, group, glu, splits, part, cnt,
+                             stream);
+}
+
+/* scratch of the prefill GEMM's activation pass: prepared rows, step sums */
+static size_t w4_prep_bytes(size_t M, size_t K) {
+    return ((M * K * sizeof(uint16_t) + 255) & ~(size_t)255) + (K / 128) * snx_w4_prep_rows(M) * sizeof(float);
+}
+
+/* Whether M x N x K runs the prefill GEMM in `splits` spans (1 for the SwiGLU
+ * form): where it may and the batch kernel is not estimated to be faster.
+ * Below SNX_W4_GEMM_MIN_M only where the allocation-free entry point, which
+ * decides alike, has the scratch for it. */
+static int w4_takes_gemm(size_t M, size_t N, size_t K, int group, const uint16_t* scales, const uint32_t* qzeros,
+                         int y_f32, int splits) {
+    if (M < (y_f32 ? SNX_W4_GEMM_MIN_M : SNX_W4_GEMM_MIN_M_BF16) || ((uintptr_t)scales & 3u) != 0 ||
+        ((uintptr_t)qzeros & 3u) != 0 || !snx_w4a16_gemm_ok(M, N, K, group) ||
+        (M < SNX_W4_GEMM_MIN_M && w4_prep_bytes(M, K) > SNEPPX_NOALLOC_SCRATCH_BYTES))
+        return 0;
+    return !snx_w4a16_batch_ok(M, N, K, group, scales, qzeros) ||
+           snx_w4a16_gemm_cost(M, N, K, splits) <= snx_w4a16_batch_cost(M, N, K);
+}
+
+/* The scratch that SNEPPX_qlinear_w4a16_noalloc is documented to need:
+ * prepared activations from SNX_W4_GEMM_MIN_M rows on, split-K partials for
+ * the decode shapes outside the persistent small-M kernel. */
+static size_t w4_noalloc_bytes(size_t M, size_t N, size_t K, int group, const uint16_t* scales,
+                               const uint32_t* qzeros) {
+    const int words = ((uintptr_t)scales & 3u) == 0 && ((uintptr_t)qzeros & 3u) == 0;
+    if (M >= SNX_W4_GEMM_MIN_M && words && snx_w4a16_gemm_ok(M, N, K, group)) return w4_prep_bytes(M, K);
+    const int kspan = snx_w4a16_splitk_span(M, K, group);
+    if (kspan && !(words && snx_w4a16_mt_ok(M, K, group, 0)) &&
+        (M > 4 || (M > 1 && !snx_w4a16_small_ok(M, K, group, 0))))
+        return K / (size_t)kspan * M * N * sizeof(float);
+    return 0;
+}
+
 static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const uint32_t* qweight,
                         const uint16_t* scales, const uint32_t* qzeros, const int32_t* g_idx,
                         size_t G, const float* bias, void* y, SNEPPXDtype y_dtype, size_t M,
@@ -140,13 +195,16 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
         G = K / (size_t)group;
     }
     snx_clear_error();
-    if (!g_idx && M >= SNX_W4_GEMM_MIN_M && aligned16(x) && aligned16(qweight) &&
-        ((uintptr_t)scales & 3u) == 0 && ((uintptr_t)qzeros & 3u) == 0 &&
-        snx_w4a16_gemm_ok(M, N, K, group)) {
+    const int aligned = !g_idx && aligned16(x) && aligned16(qweight);
+    /* the allocation-free entry point's limit is the one its header gives, also
+     * where the batch kernel would need less */
+    if (noalloc && aligned && !snx_noalloc_scratch(w4_noalloc_bytes(M, N, K, group, scales, qzeros), who)) return -1;
+    if (aligned && w4_takes_gemm(M, N, K, group, scales, qzeros, y_f32,
+                                 snx_w4a16_gemm_splits(M, N, K))) {
         /* prefill GEMM: activations prepared once into the call's scratch */
         const size_t Mp = snx_w4_prep_rows(M);
         const size_t xp_bytes = (M * K * sizeof(uint16_t) + 255) & ~(size_t)255;
-        char* ws = (char*)w4_scratch(xp_bytes + (K / 128) * Mp * sizeof(float), noalloc, stream);
+        char* ws = (char*)w4_scratch(w4_prep_bytes(M, K), noalloc, stream);
         if (!ws) return -1;
         uint16_t* xp = (uint16_t*)ws;
         float* xs = (float*)(ws + xp_bytes);
@@ -170,6 +228,12 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
         /* 2 <= M <= 16: one persistent workgroup per CU, activations staged once */
         return snx_k_w4a16_gemv_mt(x, qweight, scales, qzeros, NULL, y, bias, y_f32, M, N, K, stream);
     }
+    /* M <= 4 within the LDS-staged small-M kernel (groups of 256 and more):
+     * 7.3 and 8.1 us at M = 1, 2 (N = 6144, K = 4096), the batch kernel 9.4 */
+    const int small = M == 1 ? snx_w4a16_gemv1_ok(1, K, group, scales, qzeros) || snx_w4a16_small_ok(1, K, group, 0)
+                             : M <= 4 && snx_w4a16_small_ok(M, K, group, 0);
+    if (aligned && !small && snx_w4a16_batch_ok(M, N, K, group, scales, qzeros))
+        return w4_batch(who, noalloc, x, qweight, scales, qzeros, bias, y, y_f32, M, N, K, group, 0, stream);
     const int kspan = snx_w4a16_splitk_span(M, K, group);
     if (!g_idx && (M > 4 || (M > 1 && !snx_w4a16_small_ok(M, K, group, 0))) && kspan &&
         aligned16(x) && aligned16(qweight)) {
@@ -300,12 +364,11 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
             group, K);
     REQUIRE(aligned16(out), "qlinear_w4a16_swiglu: out must be 16-byte aligned");
     snx_clear_error();
-    if (M >= SNX_W4_GEMM_MIN_M && aligned16(x) && aligned16(qweight) &&
-        ((uintptr_t)scales & 3u) == 0 && ((uintptr_t)qzeros & 3u) == 0 &&
-        snx_w4a16_gemm_ok(M, 2 * F, K, group)) {
+    const int aligned = aligned16(x) && aligned16(qweight);
+    if (aligned && w4_takes_gemm(M, 2 * F, K, group, scales, qzeros, 0, 1)) {
         const size_t Mp = snx_w4_prep_rows(M);
         const size_t xp_bytes = (M * K * sizeof(uint16_t) + 255) & ~(size_t)255;
-        char* ws = (char*)snx_workspace(xp_bytes + (K / 128) * Mp * sizeof(float), 1, stream);
+        char* ws = (char*)snx_workspace(w4_prep_bytes(M, K), 1, stream);
         if (!ws) return -1;
         uint16_t* xp = (uint16_t*)ws;
         float* xs = (float*)(ws + xp_bytes);
@@ -318,7 +381,12 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
     if (M == 1 && aligned16(x) && aligned16(qweight) &&
         snx_w4a16_gemv1_swiglu_ok(F, K, group, scales, qzeros))
         return snx_k_w4a16_gemv1_swiglu(x, qweight, scales, qzeros, bias, out, F, K, group, stream);
-    /* other decode rows: the [M][2F] projection in fp32 scratch, then the same rule */
+    /* (up to 8 rows of the persistent decode kernel's shapes its fp32 rows and
+     * the rule's own pass stay faster: 20.8 against 22.5 us at F = 14336) */
+    if (aligned && !(M <= 8 && snx_w4a16_mt_ok(M, K, group, 0)) &&
+        snx_w4a16_batch_ok(M, 2 * F, K, group, scales, qzeros))
+        return w4_batch("qlinear_w4a16_swiglu", 0, x, qweight, scales, qzeros, bias, out, 0, M, F, K, group, 1, stream);
+    /* other shapes: the [M][2F] projection in fp32 scratch, then the same rule */
     float* gu = (float*)snx_workspace(M * 2 * F * sizeof(float), 0, stream);
     if (!gu) return -1;
     int rc = SNEPPX_qlinear_w4a16(x, qweight, scales, qzeros, NULL, 0, bias, gu, SNEPPX_FLOAT32, M,
@@ -343,11 +411,10 @@ int SNEPPX_qlinear_w4a16_mlp(const uint16_t* x, const uint32_t* gu_qweight, cons
     REQUIRE(y_dtype == SNEPPX_BFLOAT16 || y_dtype == SNEPPX_FLOAT32,
             "qlinear_w4a16_mlp: y_dtype must be SNEPPX_BFLOAT16 or SNEPPX_FLOAT32");
     snx_clear_error();
-    const int aligned = aligned16(x) && aligned16(gu_qweight) && aligned16(dn_qweight) &&
-                        ((uintptr_t)gu_scales & 3u) == 0 && ((uintptr_t)gu_qzeros & 3u) == 0 &&
-                        ((uintptr_t)dn_scales & 3u) == 0 && ((uintptr_t)dn_qzeros & 3u) == 0;
-    if (M >= SNX_W4_GEMM_MIN_M && aligned && F % 128 == 0 && snx_w4a16_gemm_ok(M, 2 * F, H, group) &&
-        snx_w4a16_gemm_ok(M, N, F, group)) {
+    if (aligned16(x) && aligned16(gu_qweight) && aligned16(dn_qweight) && F % 128 == 0 &&
+        w4_takes_gemm(M, 2 * F, H, group, gu_scales, gu_qzeros, 0, 1) &&
+        w4_takes_gemm(M, N, F, group, dn_scales, dn_qzeros, y_dtype == SNEPPX_FLOAT32,
+                      snx_w4a16_gemm_splits(M, N, F))) {
         /* x prepared once; the gate/up GEMM's SwiGLU epilogue writes the down
          * GEMM's prepared input (slot order + step sums) */
         const size_t Mp = snx_w4_prep_rows(M);

@@ -29,6 +29,8 @@ long snx_workspace_count(void);
 /* the current device's static scratch array (noalloc.hip) when `bytes` fit
  * in it, else NULL with the error text set (prefixed by `who`) */
 void* snx_noalloc_scratch(size_t bytes, const char* who);
+/* its static arrival counters: zero, and left zero by every call */
+void* snx_noalloc_counters(size_t bytes, const char* who);
 void snx_clear_error(void);
 int snx_launch_check(const char* kernel);
 
@@ -189,6 +191,20 @@ int snx_k_w4a16_generic(const uint16_t* x, const uint32_t* qw, const uint16_t* s
                         void* stream);
 int snx_w4a16_gemv_supported(size_t M, size_t N, size_t K, int group);
 
+/* W4A16 decode batches (w4_batch_kernels.hip): K % 128 == 0, groups a power
+ * of two from 32 on.  K in `splits` spans; the partials and the arrival
+ * counters (zero when taken, left zero) that a call with splits > 1 takes;
+ * the estimated time in 0.1 us.  glu: qw the stacked [2N][K] gate/up rows, y
+ * bf16 [M][N] = silu(gate) * up, splits / part / cnt those of 2N. */
+int snx_w4a16_batch_ok(size_t M, size_t N, size_t K, int group, const void* scales, const void* qzeros);
+int snx_w4a16_batch_splits(size_t M, size_t N, size_t K);
+size_t snx_w4a16_batch_cost(size_t M, size_t N, size_t K);
+size_t snx_w4a16_batch_part_bytes(size_t M, size_t N, int splits);
+size_t snx_w4a16_batch_cnt_bytes(size_t M, size_t N);
+int snx_k_w4a16_batch(const uint16_t* x, const uint32_t* qw, const uint16_t* scales, const uint32_t* qzeros,
+                      void* y, const float* bias, int y_f32, size_t M, size_t N, size_t K, int group, int glu,
+                      int splits, void* part, uint32_t* cnt, void* stream);
+
 /* W4A16 prefill GEMM (w4_gemm_kernels.hip): activations prepared once
  * (k-slot order + fp32 sums per 128 columns, xs [K/128][Mp]), then the GEMM. */
 size_t snx_w4_prep_rows(size_t M);
@@ -199,6 +215,7 @@ int snx_k_w4_prep_x(const uint16_t* x, uint16_t* xp, float* xs, size_t M, size_t
  * the partials / counters workspaces a call with `splits` > 1 takes (the
  * counters zero when taken; every call leaves them zero) */
 int snx_w4a16_gemm_splits(size_t M, size_t N, size_t K);
+size_t snx_w4a16_gemm_cost(size_t M, size_t N, size_t K, int splits);
 size_t snx_w4a16_gemm_part_bytes(size_t M, size_t N, int splits);
 size_t snx_w4a16_gemm_cnt_bytes(size_t M, size_t N);
 int snx_k_w4a16_gemm(const uint16_t* xp, const float* xs, const uint32_t* qw,
