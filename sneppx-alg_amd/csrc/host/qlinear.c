@@ -116,6 +116,19 @@ int SNEPPX_qlinear_w8_gemv(const float* x, const int8_t* qweight, const float* s
     REQUIRE(K % 16 != 0 || (aligned16(x) && aligned16(qweight)),
             "qlinear_w8_gemv: x and qweight must be 16-byte aligned");
     snx_clear_error();
+    if (snx_w8_batch_ok(M, N, K, qweight)) {
+        const int splits = snx_w8_batch_splits(M, N, K);
+        void* xp = snx_workspace(snx_w8_batch_xp_bytes(M, K), 1, stream);
+        void* part = NULL;
+        uint32_t* cnt = NULL;
+        if (!xp) return -1;
+        if (splits > 1) {
+            part = snx_workspace(snx_w8_batch_part_bytes(M, N, splits), 3, stream);
+            cnt = (uint32_t*)snx_workspace_zeroed(snx_w8_batch_cnt_bytes(M, N), 4, stream);
+            if (!part || !cnt) return -1;
+        }
+        return snx_k_w8_batch(x, qweight, scales, y, bias, M, N, K, splits, xp, part, cnt, stream);
+    }
     return snx_k_w8_gemv(x, qweight, scales, y, bias, M, N, K, stream);
 }
 

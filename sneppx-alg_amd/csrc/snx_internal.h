@@ -149,6 +149,16 @@ int snx_k_w4_gptq_quantize(const float* w, const int32_t* g_idx, size_t G, uint3
 /* bias (fp32 [N] or NULL) is added to the fp32 result of every linear below */
 int snx_k_w8_gemv(const float* x, const int8_t* q, const float* s, float* y, const float* bias,
                   size_t M, size_t N, size_t K, void* stream);
+/* the same for M >= 2 on the matrix cores (w8_batch_kernels.hip): x in three
+ * bf16 pieces (xp), K in `splits` spans (partials, and counters that are zero
+ * when taken and left zero, with splits > 1) */
+int snx_w8_batch_ok(size_t M, size_t N, size_t K, const void* q);
+size_t snx_w8_batch_xp_bytes(size_t M, size_t K);
+int snx_w8_batch_splits(size_t M, size_t N, size_t K);
+size_t snx_w8_batch_part_bytes(size_t M, size_t N, int splits);
+size_t snx_w8_batch_cnt_bytes(size_t M, size_t N);
+int snx_k_w8_batch(const float* x, const int8_t* q, const float* s, float* y, const float* bias, size_t M, size_t N,
+                   size_t K, int splits, void* xp, void* part, uint32_t* cnt, void* stream);
 /* y_f32: 1 -> fp32 output, 0 -> bf16.  perm (uint16 [K], may be NULL): the
  * weight columns are stored in that order (M <= 4 only, see small_ok). */
 int snx_k_w4a16_gemv(const uint16_t* x, const uint32_t* qw, const uint16_t* scales,
