@@ -219,8 +219,8 @@ __global__ void __launch_bounds__(256) k_w8_gemv_any(const float* __restrict__ x
 }
 
 // -------------------------------------------------------------- W4A16 GEMV
-// (M > 4 and outside the batch kernel: an odd number of scales, scales or zero
-// words off their 4-byte alignment, operands past its 31-bit offsets.)
+// (M > 4 and outside the batch kernel: scales or zero words off their 4-byte
+// alignment, operands past its 31-bit offsets.)
 // Work: a workgroup owns 16 output columns n and all of K; its 4 waves take
 // one quarter of K each and meet in LDS.  Per 128-column step a lane loads
 // the 16 bytes (32 nibbles) of row n0 + lane%16 at column 32*(lane/16), which

@@ -169,6 +169,16 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
     }
     const int ncol = c0 + (lane & 31), nc = n0 + (ncol < N ? ncol : N - 1);
     const uint32_t srow = (uint32_t)nc * G, zrow = (uint32_t)nc * ZW;
+    // an odd number of scales has a last one that no aligned word within the
+    // array holds: read by itself, by every wave (only groups of 128 and more
+    // can leave an odd number)
+    const uint32_t total = (uint32_t)(glu ? 2 * N : N) * G, lastw = (total & ~1u) - 2u;
+    // (made scalar here, so that no wait for it sits among the loop's loads);
+    // glast: its group, none where the number is even
+    const uint32_t glast = total & 1u ? G - 1 : ~0u;
+    const int last_row = (glu ? 2 * N : N) - 1;
+    const float slast = GS == 128 && (total & 1u)
+                            ? f16_dev((uint16_t)__builtin_amdgcn_readfirstlane(scales[total - 1])) : 0.0f;
 
     auto issue = [&](int slot, int t) {
         uint8_t* st = ring + slot * STAGE;
@@ -181,7 +191,7 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
         // of units 0, 1 in lanes 0..31 and of units 2, 3 in lanes 32..63)
         const uint32_t g = ((uint32_t)kt * BK) >> gshift;
         const uint32_t si = srow + g + (GS == 32 ? 2u * (uint32_t)(lane >> 5) : 0u);
-        lds_load4(rs, st + SA + OFF_S + nw * 256, (si & ~1u) * 2u);
+        lds_load4(rs, st + SA + OFF_S + nw * 256, ((si & ~1u) < lastw ? si & ~1u : lastw) * 2u);
         // without zero points the slot is filled and never read
         lds_load4(rz, st + SA + OFF_Z + nw * 256, qz ? (zrow + (g >> 3)) * 4u : 0u);
     };
@@ -308,6 +318,7 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
                     const uint32_t word = GS == 32 ? sw[s][u >> 1] : sw[s][0];
                     zc[u][s] = qz ? (zw[s] >> (4 * ((gq + (GS == 128 ? 0 : u)) & 7))) & 15u : 8u;
                     sc[u][s] = f16_dev((uint16_t)(word >> (16 * half)));
+                    if (GS == 128 && gq == glast && n0 + n >= last_row) sc[u][s] = slast;
                 }
 #pragma unroll
             for (int j = 0; j < J - 1; j++) {
@@ -538,7 +549,7 @@ int snx_w4a16_batch_ok(size_t M, size_t N, size_t K, int group, const void* scal
     if (M < 1 || K % BK != 0 || group < 32 || (group & (group - 1)) != 0 || K % (size_t)group != 0) return 0;
     const size_t G = K / (size_t)group;
     // scales are read as aligned words of two; 31-bit buffer offsets
-    return (N * G) % 2 == 0 && ((uintptr_t)scales & 3u) == 0 && ((uintptr_t)qz & 3u) == 0 &&
+    return N * G >= 2 && ((uintptr_t)scales & 3u) == 0 && ((uintptr_t)qz & 3u) == 0 &&
            M * K * 2 < (1ull << 31) && N * K / 2 < (1ull << 31) && N * G * 2 < (1ull << 31) &&
            (M + 96) * N * 4 < (1ull << 31) && M <= 96 * 65535ull;
 }
