@@ -1330,7 +1330,10 @@ int snx_k_i8_gemm(const int8_t* A, const int8_t* W, const float* sA, const float
         snx_set_error("i8 gemm: K=%zu must be a multiple of 16", K);
         return -1;
     }
-    if (K % TBK == 0 && M >= 128 && N >= 128) {
+    const bool tiled = K % TBK == 0 && M >= 128 && N >= 128;
+    if (!c_i32 && (tiled ? snx_q8_batch_better(0, M, N, K) : snx_q8_batch_ok(0, M, N, K)))
+        return snx_k_q8_batch(0, A, sA, W, sW, out_bf16, bias, 0, M, N, K, st);
+    if (tiled) {
         // the persistent kernel addresses operands with 31-bit buffer offsets
         // and writes bf16 output in 16-byte row pieces
         const bool fits = (uint64_t)M * K < (1ull << 31) && (uint64_t)N * K < (1ull << 31);
@@ -1383,6 +1386,8 @@ int snx_k_mx8_gemm(const uint8_t* A, const int8_t* sA, const uint8_t* W, const i
         snx_set_error("mx gemm: K %% 128 == 0 and operands below 4 GiB are required");
         return -1;
     }
+    if (snx_q8_batch_better(2 + mf, M, N, K))
+        return snx_k_q8_batch(2 + mf, A, sA, W, sW, out, nullptr, y_f32, M, N, K, st);
     const int m = (int)M, n = (int)N, k = (int)K;
 #define SNX_MX8(F, B)                                                                       \
     return y_f32 ? launch_mx8_tiled<F, B, true>(A, sA, W, sW, out, m, n, k, S(st))          \
@@ -1402,7 +1407,10 @@ int snx_k_fp8_gemm(const uint8_t* A, const uint8_t* W, const float* sA, const fl
         snx_set_error("fp8 gemm: K=%zu must be a multiple of 32", K);
         return -1;
     }
-    if (K % TBK == 0 && M >= 128 && N >= 128) {
+    const bool tiled = K % TBK == 0 && M >= 128 && N >= 128;
+    if (tiled ? snx_q8_batch_better(1, M, N, K) : snx_q8_batch_ok(1, M, N, K))
+        return snx_k_q8_batch(1, A, sA, W, sW, out_bf16, bias, 0, M, N, K, st);
+    if (tiled) {
         const int8_t* a8 = reinterpret_cast<const int8_t*>(A);
         const int8_t* w8 = reinterpret_cast<const int8_t*>(W);
         if (N % 8 == 0 && (reinterpret_cast<uintptr_t>(out_bf16) & 15) == 0 && (uint64_t)M * N * 2 < BUF_DROP &&

@@ -254,6 +254,13 @@ int snx_k_w4a16_gemm_swiglu_prep(const uint16_t* xp, const float* xs, const uint
                                  float* out_xs, const float* bias, size_t M, size_t F, size_t K, int group,
                                  size_t Mp, void* stream);
 
+/* few rows of int8 / fp8 / MX operands (q8_batch_kernels.hip).  kind: 0 int8
+ * (fp32 sA [M], sW [N]), 1 fp8 (fp32 sA[0], sW[0]), 2 + MFMA element format: MX
+ * (int8 exponents [rows][K / 32], 4-byte aligned) */
+int snx_q8_batch_ok(int kind, size_t M, size_t N, size_t K);
+int snx_q8_batch_better(int kind, size_t M, size_t N, size_t K);
+int snx_k_q8_batch(int kind, const void* A, const void* sA, const void* W, const void* sW, void* out,
+                   const float* bias, int y_f32, size_t M, size_t N, size_t K, void* stream);
 int snx_k_i8_gemm(const int8_t* A, const int8_t* W, const float* sA, const float* sW,
                   int32_t* c_i32, uint16_t* out_bf16, const float* bias, size_t M, size_t N,
                   size_t K, void* stream);
