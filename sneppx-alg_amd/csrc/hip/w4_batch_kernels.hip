@@ -554,29 +554,37 @@ int snx_w4a16_batch_ok(size_t M, size_t N, size_t K, int group, const void* scal
            (M + 96) * N * 4 < (1ull << 31) && M <= 96 * 65535ull;
 }
 
-// Spans of K: as many as make the tiles fill the CUs (one workgroup's LDS is
-// most of a CU's), each at least two steps for every wave group.  Measured at
-// N = 6144, K = 4096, M = 16: 1 span 17.9, 2 13.3, 4 10.5, 5 9.7, 6 (288
-// workgroups, more than the CUs) 13.1 us.
+// Spans of K: as many as the CUs take at once (one workgroup's LDS is most of
+// a CU's), and no more than pay: a span takes its share off the steps and adds
+// its results to the meeting; the best counts measured lie near sqrt(4/3
+// steps), and K = 512 stays whole (N = 1792, M = 8: 4.5 us, 2 spans 5.8).  64
+// rows and more meet four spans at a time.
+// N = 6144, K = 4096, M = 16: 1 span 17.9 us, 2 13.3, 4 10.5, 5 9.7, 6 (288
+// workgroups, more than the CUs) 13.1; N = 961, M = 8: K = 2048 1 span 10.3, 2
+// 9.0, 4 7.4, 6 7.0, 8 7.7; K = 8192 4 spans 14.4, 8 11.6, 12 11.7, 16 12.5.
 int snx_w4a16_batch_splits(size_t M, size_t N, size_t K) {
-    const size_t rows = (size_t)rows_of((int)M), ncu = (size_t)snx::cu_count();
-    const size_t units = ((N + BN - 1) / BN) * ((M + rows - 1) / rows), most = K / BK / (2 * KW);
+    const size_t rows = (size_t)rows_of((int)M), ncu = (size_t)snx::cu_count(), steps = K / BK;
+    const size_t units = ((N + BN - 1) / BN) * ((M + rows - 1) / rows), most = steps < 8 ? 1 : steps / KW;
     size_t s = ncu / units;
     if (s > most) s = most;
+    while (s > 1 && 3 * s * (s - 1) >= 4 * steps) s--;
+    if (rows >= 64 && s > 4) s -= s % 4;
     return s < 1 ? 1 : (int)s;
 }
 
 // Estimated time in units of 0.1 us, to set against the prefill GEMM's: a
-// fixed part, 2.5 us for the meeting of the spans, and the steps of a wave
-// group (0.87 us with 16 rows, 0.95, 1.6 and 2.0 with 32, 64 and 96) per
-// round of the CUs.
+// fixed part, the meeting of the spans, and for each round of the CUs its
+// start and the steps of a wave group (0.9 us with 16 rows, 1.0, 1.6 and 2.2
+// with 32, 64 and 96).  N = 7168, K = 3584 at M = 320, 394, 1049 (1, 2, 3
+// rounds): 35.4, 65.0, 100 us measured, 35.3, 68.6, 102 estimated.
 size_t snx_w4a16_batch_cost(size_t M, size_t N, size_t K) {
     const int rows = rows_of((int)M), splits = snx_w4a16_batch_splits(M, N, K);
     const size_t ncu = (size_t)snx::cu_count();
     const size_t units = ((N + BN - 1) / BN) * ((M + rows - 1) / rows) * splits;
     const size_t steps = (K / BK + (size_t)splits * KW - 1) / ((size_t)splits * KW);
-    const size_t step = rows == 16 ? 9 : rows == 32 ? 10 : rows == 64 ? 16 : 20;
-    return 40 + (splits > 1 ? 25 : 0) + (units + ncu - 1) / ncu * steps * step;
+    const size_t step = rows == 16 ? 9 : rows == 32 ? 10 : rows == 64 ? 16 : 22;
+    const size_t meet = splits == 1 ? 0 : rows < 96 ? 25 : 20 + 10 * (size_t)splits;
+    return 20 + meet + (units + ncu - 1) / ncu * (25 + steps * step);
 }
 
 size_t snx_w4a16_batch_part_bytes(size_t M, size_t N, int splits) {

@@ -812,13 +812,15 @@ int snx_w4a16_gemm_splits(size_t M, size_t N, size_t K) {
 }
 
 // Estimated time in units of 0.1 us, to set against the batch kernel's: the
-// activation pass and the kernel's fixed parts (16 us), and 1.6 us a step for
-// every round of the CUs.  splits: the K spans the call runs.
+// activation pass (1 us per 10^6 elements), the kernel's fixed parts (10 us, 16
+// where spans meet) and 1.6 us a step for every round of the CUs.  splits: the
+// K spans the call runs.  N = 7168, K = 3584 at M = 320, 768, 1049: 38.7, 54.4,
+// 61.4 us measured, 39.5, 57.4, 58.6 estimated.
 size_t snx_w4a16_gemm_cost(size_t M, size_t N, size_t K, int splits) {
     const size_t ntiles = ((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN);
     const size_t ncu = (size_t)snx::cu_count(), nk = K / GBK;
     const size_t full = ntiles / ncu, rem = ntiles % ncu;
-    return 160 + 16 * (full * nk + (rem ? nk / (size_t)splits : 0));
+    return (splits > 1 ? 160 : 100) + M * K / 100000 + 16 * (full * nk + (rem ? nk / (size_t)splits : 0));
 }
 
 // Bytes of the span partials (`part`) and arrival counters (`cnt`) of a

@@ -164,7 +164,8 @@ static size_t w4_prep_bytes(size_t M, size_t K) {
 }
 
 /* Whether M x N x K runs the prefill GEMM in `splits` spans (1 for the SwiGLU
- * form): where it may and the batch kernel is not estimated to be faster.
+ * form): where it may and the batch kernel is not estimated to be faster by a
+ * tenth (what the estimates are off by).
  * Below SNX_W4_GEMM_MIN_M only where the allocation-free entry point, which
  * decides alike, has the scratch for it. */
 static int w4_takes_gemm(size_t M, size_t N, size_t K, int group, const uint16_t* scales, const uint32_t* qzeros,
@@ -174,7 +175,28 @@ static int w4_takes_gemm(size_t M, size_t N, size_t K, int group, const uint16_t
         (M < SNX_W4_GEMM_MIN_M && w4_prep_bytes(M, K) > SNEPPX_NOALLOC_SCRATCH_BYTES))
         return 0;
     return !snx_w4a16_batch_ok(M, N, K, group, scales, qzeros) ||
-           snx_w4a16_gemm_cost(M, N, K, splits) <= snx_w4a16_batch_cost(M, N, K);
+           10 * snx_w4a16_gemm_cost(M, N, K, splits) <= 11 * snx_w4a16_batch_cost(M, N, K);
+}
+
+/* One row, and M <= 4 within the LDS-staged small-M kernel (groups of 256 and
+ * more): 7.3 and 8.1 us at M = 1, 2 (N = 6144, K = 4096), the batch kernel
+ * 9.4; stacked gate/up rows and their SwiGLU at M = 1, F = 1408, K = 1792: 5.1
+ * and 8.2. */
+static int w4_small(size_t M, size_t K, int group, const uint16_t* scales, const uint32_t* qzeros) {
+    return M == 1 ? snx_w4a16_gemv1_ok(1, K, group, scales, qzeros) || snx_w4a16_small_ok(1, K, group, 0)
+                  : M <= 4 && snx_w4a16_small_ok(M, K, group, 0);
+}
+
+/* Shapes with little to stream, where the start and the meeting of the batch
+ * kernel's spans weigh most.  17 to 32 rows with K up to 1024: the decode GEMV,
+ * 4.3 against 5.0 us at N = 4096, K = 512, M = 32 and 6.1 against 7.6 at K =
+ * 1024 (N = 14336, K = 512: 7.8 against 5.8).  2 to 16 rows with K from 8192 in
+ * few split-K spans and N up to 1536: split-K, 11.2 against 12.7 us at N = 1408,
+ * K = 8192, M = 8 and 12.3 against 13.4 at N = 961, K = 13312 (N = 2048: 15.0
+ * against 14.1; in spans of 256, K = 11008: 23.4 against 12.8). */
+static int w4_short(size_t M, size_t N, size_t K, int group) {
+    return M > 16 ? M <= 32 && K <= 1024 && N <= 4096 && snx_w4a16_gemv_supported(M, N, K, group)
+                  : M > 1 && K >= 8192 && N <= 1536 && snx_w4a16_splitk_span(M, K, group) >= 512;
 }
 
 /* The scratch that SNEPPX_qlinear_w4a16_noalloc is documented to need:
@@ -241,11 +263,8 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
         /* 2 <= M <= 16: one persistent workgroup per CU, activations staged once */
         return snx_k_w4a16_gemv_mt(x, qweight, scales, qzeros, NULL, y, bias, y_f32, M, N, K, stream);
     }
-    /* M <= 4 within the LDS-staged small-M kernel (groups of 256 and more):
-     * 7.3 and 8.1 us at M = 1, 2 (N = 6144, K = 4096), the batch kernel 9.4 */
-    const int small = M == 1 ? snx_w4a16_gemv1_ok(1, K, group, scales, qzeros) || snx_w4a16_small_ok(1, K, group, 0)
-                             : M <= 4 && snx_w4a16_small_ok(M, K, group, 0);
-    if (aligned && !small && snx_w4a16_batch_ok(M, N, K, group, scales, qzeros))
+    if (aligned && !w4_small(M, K, group, scales, qzeros) && !w4_short(M, N, K, group) &&
+        snx_w4a16_batch_ok(M, N, K, group, scales, qzeros))
         return w4_batch(who, noalloc, x, qweight, scales, qzeros, bias, y, y_f32, M, N, K, group, 0, stream);
     const int kspan = snx_w4a16_splitk_span(M, K, group);
     if (!g_idx && (M > 4 || (M > 1 && !snx_w4a16_small_ok(M, K, group, 0))) && kspan &&
@@ -396,7 +415,8 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
         return snx_k_w4a16_gemv1_swiglu(x, qweight, scales, qzeros, bias, out, F, K, group, stream);
     /* (up to 8 rows of the persistent decode kernel's shapes its fp32 rows and
      * the rule's own pass stay faster: 20.8 against 22.5 us at F = 14336) */
-    if (aligned && !(M <= 8 && snx_w4a16_mt_ok(M, K, group, 0)) &&
+    if (aligned && !(M <= 8 && snx_w4a16_mt_ok(M, K, group, 0)) && !(M == 1 && w4_small(M, K, group, scales, qzeros)) &&
+        !w4_short(M, 2 * F, K, group) &&
         snx_w4a16_batch_ok(M, 2 * F, K, group, scales, qzeros))
         return w4_batch("qlinear_w4a16_swiglu", 0, x, qweight, scales, qzeros, bias, out, 0, M, F, K, group, 1, stream);
     /* other shapes: the [M][2F] projection in fp32 scratch, then the same rule */
