@@ -34,11 +34,11 @@ struct Fmt {
 };
 
 // f: 0 e4m3, 1 e5m2, 2 e3m2, 3 e2m3, 4 e2m1 (rows of the tie tables)
-__host__ __device__ inline Fmt fmt_of(int f) {
+__host__ __device__ constexpr Fmt fmt_of(int f) {
     const int mb = f == 0 ? 3 : f == 1 ? 2 : f == 2 ? 2 : f == 3 ? 3 : 1;
     const int eb = f == 0 ? 4 : f == 1 ? 5 : f == 2 ? 3 : f == 3 ? 2 : 2;
     const int bias = f == 0 ? 7 : f == 1 ? 15 : f == 2 ? 3 : 1;
-    Fmt F;
+    Fmt F{};
     F.mb = mb;
     F.bits = 1 + eb + mb;
     F.bias = bias;
@@ -192,6 +192,76 @@ __global__ void __launch_bounds__(256) k_mx_quant_blocks(const float* __restrict
         out.put(nonfinite ? encode_nonfinite(v, F) : encode(v, s, F), F.bits);
     }
     out.flush();
+}
+
+// ---- blocks of 32 of whole rows: four lanes per block --------------------
+// Bound by the 4-byte reads.  A lane holds 8 elements (two 16-byte loads) and
+// writes its 8 codes at once; the peak meets by DPP within the quad, and the
+// format is a template argument, so an element is a dozen 32-bit operations on
+// v = x * 2^-s (exact, or so far below the format's range that it rounds to 0
+// either way).  512 x 4096 E4M3: 28 us with k_mx_quant_blocks, 5.9
+// here (2 us at the rate of a large copy).
+template <int CTRL>
+__device__ inline uint32_t quad_max(uint32_t v) {
+    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+    return o > v ? o : v;
+}
+
+template <int FI>
+__global__ void __launch_bounds__(256) k_mx_quant32(const float* __restrict__ x,
+                                                    uint8_t* __restrict__ packed,
+                                                    int8_t* __restrict__ scales, size_t nblocks) {
+    constexpr Fmt F = fmt_of(FI);
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= nblocks * 4) return;   // whole quads
+    const u32x4 lo = reinterpret_cast<const u32x4*>(x)[2 * t], hi = reinterpret_cast<const u32x4*>(x)[2 * t + 1];
+    const uint32_t b[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    uint32_t peak = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint32_t a = b[i] & 0x7FFFFFFFu;   // ordered as |x|, infinities and NaN above
+        peak = a > peak ? a : peak;
+    }
+    peak = quad_max<0x4E>(quad_max<0xB1>(peak));
+    const bool finite = peak < 0x7F800000u;
+    const int s = finite ? scale_of(peak ? peak : 0x3F800000u, F, false) : 0;
+    if ((t & 3) == 0) scales[t >> 2] = (int8_t)(uint8_t)(uint32_t)s;   // int8 cast wraps
+    uint64_t out = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        uint32_t c;
+        if (finite) {
+            const float v = fabsf(ldexpf(__builtin_bit_cast(float, b[i]), -s));
+            const uint32_t vb = __builtin_bit_cast(uint32_t, v);
+            const int ev = (int)(vb >> 23) - 127;
+            constexpr int sh = 23 - F.mb;
+            const uint32_t man = vb & 0x7FFFFFu;
+            uint32_t m = (man + ((1u << (sh - 1)) - 1) + ((man >> sh) & 1u)) >> sh;
+            uint32_t field = (uint32_t)(ev + F.bias);
+            if (ev <= -F.bias) {
+                m = (uint32_t)rintf(v * (float)(1 << (F.mb + F.bias - 1)));
+                field = 0;
+            }
+            m = m > (uint32_t)F.mmax ? (uint32_t)F.mmax : m;
+            c = ev > F.E ? (uint32_t)(F.fmax << F.mb | F.mmax) : field << F.mb | m;
+            c |= (b[i] & 0x7FFFFFFFu) ? b[i] >> 31 << (F.bits - 1) : 0u;
+        } else {
+            c = encode_nonfinite(__builtin_bit_cast(float, b[i]), F);
+        }
+        out |= (uint64_t)c << (F.bits * i);
+    }
+    if (F.bits == 8) {
+        reinterpret_cast<u32x2*>(packed)[t] = u32x2{(uint32_t)out, (uint32_t)(out >> 32)};
+    } else if (F.bits == 4) {
+        reinterpret_cast<uint32_t*>(packed)[t] = (uint32_t)out;
+    } else {
+        uint16_t* p = reinterpret_cast<uint16_t*>(packed) + 3 * t;
+        p[0] = (uint16_t)out;
+        p[1] = (uint16_t)(out >> 16);
+        p[2] = (uint16_t)(out >> 32);
+    }
 }
 
 __global__ void __launch_bounds__(256) k_mx_dequant_blocks(const uint8_t* __restrict__ packed,
@@ -395,6 +465,19 @@ int snx_k_mx_quant_blocks(const float* x, uint8_t* packed, int8_t* scales, size_
     if (rows * nb >= (1ull << 38)) {
         snx_set_error("mx quantize: too many blocks");
         return -1;
+    }
+    // whole aligned blocks of 32 (and a grid below 2^31 threads)
+    if (bs == 32 && cols % 32 == 0 && ((uintptr_t)x & 15u) == 0 && ((uintptr_t)packed & 7u) == 0 &&
+        rows * nb <= (1ull << 28)) {
+        const size_t n = rows * nb;
+        switch (f) {
+            case 0: k_mx_quant32<0><<<grid_of(n * 4), 256, 0, S(st)>>>(x, packed, scales, n); break;
+            case 1: k_mx_quant32<1><<<grid_of(n * 4), 256, 0, S(st)>>>(x, packed, scales, n); break;
+            case 2: k_mx_quant32<2><<<grid_of(n * 4), 256, 0, S(st)>>>(x, packed, scales, n); break;
+            case 3: k_mx_quant32<3><<<grid_of(n * 4), 256, 0, S(st)>>>(x, packed, scales, n); break;
+            default: k_mx_quant32<4><<<grid_of(n * 4), 256, 0, S(st)>>>(x, packed, scales, n); break;
+        }
+        return snx_launch_check("k_mx_quant32");
     }
     k_mx_quant_blocks<<<grid_of(rows * nb), 256, 0, S(st)>>>(x, packed, scales, rows, cols, bs, f);
     return snx_launch_check("k_mx_quant_blocks");
