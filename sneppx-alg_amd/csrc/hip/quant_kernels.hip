@@ -671,6 +671,65 @@ __global__ void k_w4_awq_quantize(const float* __restrict__ w, uint32_t* __restr
     }
 }
 
+// The same for groups of 32, 64 and 128 with K % 32 == 0, w and qw 16-byte
+// aligned: a lane holds 8 elements (two 16-byte loads, one word of codes), so
+// w is read once and a group's extremes meet by shuffles within group / 8
+// lanes; a wave takes 512 elements a step.  Bound by the reads of w and the
+// correctly rounded divisions.  14336 x 4096,
+// groups of 128: 233 us with k_w4_awq_quantize, 63 here (51 at the rate of a large
+// copy).
+template <int LPG>
+__global__ void __launch_bounds__(256) k_w4_awq_quantize_v8(const float* __restrict__ w, uint32_t* __restrict__ qw,
+                                                            uint16_t* __restrict__ scales,
+                                                            uint32_t* __restrict__ qzeros, size_t N, int kw) {
+    extern __shared__ uint8_t zsh[];
+    const int G = kw / LPG, zw = (G + 7) / 8;
+    for (size_t n = blockIdx.x; n < N; n += gridDim.x) {
+        const float4* xr = reinterpret_cast<const float4*>(w) + n * (size_t)kw * 2;
+        for (int wd = threadIdx.x; wd < kw; wd += 256) {   // groups are whole: LPG divides kw
+            const float4 a = xr[2 * wd], b = xr[2 * wd + 1];
+            const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            float lo = INFINITY, hi = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                lo = nanless_min(lo, x[t]);
+                hi = nanless_max(hi, x[t]);
+            }
+#pragma unroll
+            for (int o = 1; o < LPG; o <<= 1) {
+                lo = nanless_min(lo, __shfl_xor(lo, o));
+                hi = nanless_max(hi, __shfl_xor(hi, o));
+            }
+            const float x0 = __shfl(x[0], (int)(threadIdx.x & 63 & ~(LPG - 1)));
+            if (x0 != x0) lo = hi = x0;
+            const bool degenerate = hi - lo < FLT_MIN;
+            uint16_t s16 = 0x3C00u;
+            int32_t z = 0;
+            uint32_t word = 0;
+            if (!degenerate) {
+                s16 = w4_scale_f16((hi - lo) / 15.0f);
+                const float s = f16_to_f32(s16);
+                z = clampi(round_i32(-lo / s), 0, 15);
+                const float zf = (float)z;
+#pragma unroll
+                for (int t = 0; t < 8; t++) word |= (uint32_t)clampi(round_i32(x[t] / s + zf), 0, 15) << (4 * t);
+            }
+            qw[n * (size_t)kw + wd] = word;
+            if (wd % LPG == 0) {
+                scales[n * (size_t)G + wd / LPG] = s16;
+                zsh[wd / LPG] = (uint8_t)z;
+            }
+        }
+        __syncthreads();
+        for (int zi = threadIdx.x; zi < zw; zi += 256) {
+            uint32_t word = 0;
+            for (int t = 0; t < 8 && zi * 8 + t < G; t++) word |= (uint32_t)zsh[zi * 8 + t] << (4 * t);
+            qzeros[n * (size_t)zw + zi] = word;
+        }
+        __syncthreads();
+    }
+}
+
 // a21 GPTQ act-order int4: block per row; group maxima and first-poisoned
 // columns through LDS atomics (order-independent), then codes per word.
 __global__ void k_w4_gptq_quantize(const float* __restrict__ w, const int32_t* __restrict__ g_idx,
@@ -923,6 +982,16 @@ int snx_k_w4_awq_quantize(const float* w, uint32_t* qw, uint16_t* scales, uint32
                           size_t N, size_t K, int group, void* st) {
     size_t G = K / (size_t)group;
     int grid = (int)(N < 65536 ? N : 65536);
+    if ((group == 32 || group == 64 || group == 128) && ((uintptr_t)w & 15u) == 0 && K < (1u << 30)) {
+        const int kw = (int)(K / 8);
+        if (group == 32)
+            k_w4_awq_quantize_v8<4><<<grid, 256, G + 8, S(st)>>>(w, qw, scales, qzeros, N, kw);
+        else if (group == 64)
+            k_w4_awq_quantize_v8<8><<<grid, 256, G + 8, S(st)>>>(w, qw, scales, qzeros, N, kw);
+        else
+            k_w4_awq_quantize_v8<16><<<grid, 256, G + 8, S(st)>>>(w, qw, scales, qzeros, N, kw);
+        return snx_launch_check("k_w4_awq_quantize_v8");
+    }
     k_w4_awq_quantize<<<grid, kBlock, G + 8, S(st)>>>(w, qw, scales, qzeros, N, K, group);
     return snx_launch_check("k_w4_awq_quantize");
 }
