@@ -66,10 +66,21 @@ __device__ __forceinline__ float as_f32(uint16_t v) {   // bf16 bits
     return __builtin_bit_cast(float, (uint32_t)v << 16);
 }
 
-template <typename T = float>
+// V: fp32 on 16 bytes, four values per load (the last n % 4 by block 0)
+template <typename T = float, bool V = false>
 __global__ void k_absmax(const T* __restrict__ x, size_t n, float* __restrict__ part) {
     __shared__ float sh[16];
     float m = 0.0f;
+    if (V) {
+        const float4* x4 = reinterpret_cast<const float4*>(x);
+        for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n / 4;
+             i += (size_t)gridDim.x * blockDim.x) {
+            const float4 v = x4[i];
+            m = nanless_max(nanless_max(m, fabsf(v.x)), fabsf(v.y));
+            m = nanless_max(nanless_max(m, fabsf(v.z)), fabsf(v.w));
+        }
+        if (blockIdx.x == 0 && threadIdx.x < n % 4) m = nanless_max(m, fabsf(as_f32(x[n / 4 * 4 + threadIdx.x])));
+    } else
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x)
         m = nanless_max(m, fabsf(as_f32(x[i])));
@@ -232,14 +243,31 @@ __global__ void k_dequant_int4_sym(const uint8_t* __restrict__ p, float* __restr
 // correctly rounded division, not x * (1/s): for s = amax/240 the quotient
 // puts the largest element at 240 (code 0x77) in about twice as many cases,
 // where the product's 239.99998 truncates to 224.
-template <int FMT, typename T = float>
+// V: fp32 on 16 bytes and codes on 4, four values per load (the last n % 4 by
+// block 0).  With k_absmax, 14336 x 4096: 183 us one value per load, 100 here
+// (102 at the rate of a large copy).
+template <int FMT, typename T = float, bool V = false>
 __global__ void k_fp8_encode(const T* __restrict__ x, uint8_t* __restrict__ c, size_t n,
                              const float* __restrict__ rec) {
     float s = rec ? rec[0] : 1.0f;
+    auto code = [&](float a) {
+        const float v = rec ? a / s : a;
+        return (uint32_t)(FMT == 0 ? fp8_e4m3_encode(v) : fp8_e5m2_encode(v));
+    };
+    if (V) {
+        const float4* x4 = reinterpret_cast<const float4*>(x);
+        for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n / 4;
+             i += (size_t)gridDim.x * blockDim.x) {
+            const float4 v = x4[i];
+            reinterpret_cast<uint32_t*>(c)[i] = code(v.x) | code(v.y) << 8 | code(v.z) << 16 | code(v.w) << 24;
+        }
+        const size_t i = n / 4 * 4 + threadIdx.x;
+        if (blockIdx.x == 0 && i < n) c[i] = (uint8_t)code(as_f32(x[i]));
+        return;
+    }
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x) {
-        float v = rec ? as_f32(x[i]) / s : as_f32(x[i]);
-        c[i] = FMT == 0 ? fp8_e4m3_encode(v) : fp8_e5m2_encode(v);
+        c[i] = (uint8_t)code(as_f32(x[i]));
     }
 }
 
@@ -378,6 +406,57 @@ __global__ void __launch_bounds__(256) k_quant_rows_bf16_reg(const uint16_t* __r
         }
         __syncthreads();   // sh is reused by the next row's reduction
     }
+}
+
+// k_quant_int8_rows of fp32 rows in one pass: the row in registers, CH 16-byte
+// chunks (4 values) per thread, 4 codes per store; cols % 4 == 0, cols <= 1024
+// CH, x 16-byte and q 4-byte aligned.  14336 x 4096: 126 us with one value per
+// load in two passes, 55 here (57 at the rate of a large copy).
+template <bool RNE, int CH>
+__global__ void __launch_bounds__(256) k_quant_rows_f32_reg(const float* __restrict__ x, int8_t* __restrict__ q,
+                                                            float* __restrict__ scales, size_t rows, int cols) {
+    __shared__ float sh[16];
+    const int nch = cols >> 2;
+    for (size_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        const float4* xr = reinterpret_cast<const float4*>(x + r * (size_t)cols);
+        float4 v[CH];
+        float m = 0.0f;
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const int ch = threadIdx.x + 256 * c;
+            v[c] = ch < nch ? xr[ch] : float4{0.0f, 0.0f, 0.0f, 0.0f};
+            m = nanless_max(nanless_max(m, fabsf(v[c].x)), fabsf(v[c].y));
+            m = nanless_max(nanless_max(m, fabsf(v[c].z)), fabsf(v[c].w));
+        }
+        m = block_reduce(m, nanless_max, sh);
+        const float s = m < FLT_MIN ? 1.0f : m / 127.0f;
+        const float inv = 1.0f / s;
+        if (threadIdx.x == 0) scales[r] = s;
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const int ch = threadIdx.x + 256 * c;
+            if (ch >= nch) break;
+            const float e[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
+            uint32_t w = 0u;
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const float p = e[t] * inv;
+                w |= ((uint32_t)clampi(RNE ? rne_i32(p) : round_i32(p), -128, 127) & 0xFFu) << (8 * t);
+            }
+            reinterpret_cast<uint32_t*>(q + r * (size_t)cols)[ch] = w;
+        }
+        __syncthreads();   // sh is reused by the next row's reduction
+    }
+}
+
+template <bool RNE>
+void quant_rows_f32_reg(const float* x, int8_t* q, float* scales, size_t rows, int cols, int grid, hipStream_t st) {
+    if (cols <= 1024)
+        k_quant_rows_f32_reg<RNE, 1><<<grid, 256, 0, st>>>(x, q, scales, rows, cols);
+    else if (cols <= 4096)
+        k_quant_rows_f32_reg<RNE, 4><<<grid, 256, 0, st>>>(x, q, scales, rows, cols);
+    else
+        k_quant_rows_f32_reg<RNE, 16><<<grid, 256, 0, st>>>(x, q, scales, rows, cols);
 }
 
 // tensor.c:2180-2195 (SNEPPX_tensor_fake_quant): q = floorf(x * (1/scale) +
@@ -675,9 +754,8 @@ __global__ void k_w4_awq_quantize(const float* __restrict__ w, uint32_t* __restr
 // aligned: a lane holds 8 elements (two 16-byte loads, one word of codes), so
 // w is read once and a group's extremes meet by shuffles within group / 8
 // lanes; a wave takes 512 elements a step.  Bound by the reads of w and the
-// correctly rounded divisions.  14336 x 4096,
-// groups of 128: 233 us with k_w4_awq_quantize, 63 here (51 at the rate of a large
-// copy).
+// correctly rounded divisions.  14336 x 4096, groups of 128: 233 us with
+// k_w4_awq_quantize, 63 here (51 at the rate of a large copy).
 template <int LPG>
 __global__ void __launch_bounds__(256) k_w4_awq_quantize_v8(const float* __restrict__ w, uint32_t* __restrict__ qw,
                                                             uint16_t* __restrict__ scales,
@@ -799,7 +877,10 @@ float SNEPPX_fp8_e5m2_to_float(uint8_t fp8) { return fp8_e5m2_decode(fp8); }
 int snx_reduce_parts(size_t n) { return grid_for(n, kBlock * 16, kMaxParts); }
 
 int snx_k_absmax(const float* x, size_t n, float* part, int nparts, void* st) {
-    k_absmax<<<nparts, kBlock, 0, S(st)>>>(x, n, part);
+    if (((uintptr_t)x & 15u) == 0)
+        k_absmax<float, true><<<nparts, kBlock, 0, S(st)>>>(x, n, part);
+    else
+        k_absmax<<<nparts, kBlock, 0, S(st)>>>(x, n, part);
     return snx_launch_check("k_absmax");
 }
 
@@ -851,7 +932,12 @@ int snx_k_dequant_int4_sym(const uint8_t* p, float* y, size_t n, float scale, vo
 
 int snx_k_fp8_encode(const float* x, uint8_t* c, size_t n, int fmt, const float* rec, void* st) {
     if (n == 0) return 0;
-    if (fmt == 0)
+    const int v4 = (((uintptr_t)x & 15u) | ((uintptr_t)c & 3u)) == 0;
+    if (v4 && fmt == 0)
+        k_fp8_encode<0, float, true><<<grid_for(n, kBlock * 8), kBlock, 0, S(st)>>>(x, c, n, rec);
+    else if (v4)
+        k_fp8_encode<1, float, true><<<grid_for(n, kBlock * 8), kBlock, 0, S(st)>>>(x, c, n, rec);
+    else if (fmt == 0)
         k_fp8_encode<0><<<grid_for(n, kBlock * 4), kBlock, 0, S(st)>>>(x, c, n, rec);
     else
         k_fp8_encode<1><<<grid_for(n, kBlock * 4), kBlock, 0, S(st)>>>(x, c, n, rec);
@@ -870,6 +956,13 @@ int snx_k_fp8_decode(const uint8_t* c, float* y, size_t n, int fmt, void* st) {
 int snx_k_quant_int8_rows(const float* x, int8_t* q, float* scales, size_t rows, size_t cols,
                           int rne, void* st) {
     int grid = (int)(rows < 65536 ? rows : 65536);
+    if (cols % 4 == 0 && cols <= 16384 && ((uintptr_t)x & 15u) == 0 && ((uintptr_t)q & 3u) == 0) {
+        if (rne)
+            quant_rows_f32_reg<true>(x, q, scales, rows, (int)cols, grid, S(st));
+        else
+            quant_rows_f32_reg<false>(x, q, scales, rows, (int)cols, grid, S(st));
+        return snx_launch_check("k_quant_rows_f32_reg");
+    }
     if (rne)
         k_quant_int8_rows<true, float><<<grid, kBlock, 0, S(st)>>>(x, q, scales, rows, cols);
     else
