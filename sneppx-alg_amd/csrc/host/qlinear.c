@@ -163,19 +163,19 @@ static size_t w4_prep_bytes(size_t M, size_t K) {
     return ((M * K * sizeof(uint16_t) + 255) & ~(size_t)255) + (K / 128) * snx_w4_prep_rows(M) * sizeof(float);
 }
 
-/* Whether M x N x K runs the prefill GEMM in `splits` spans (1 for the SwiGLU
- * form): where it may and the batch kernel is not estimated to be faster by a
+/* Whether M x N x K runs the prefill GEMM (glu: its SwiGLU form, which does not
+ * split K): where it may and the batch kernel is not estimated to be faster by a
  * tenth (what the estimates are off by).
  * Below SNX_W4_GEMM_MIN_M only where the allocation-free entry point, which
  * decides alike, has the scratch for it. */
 static int w4_takes_gemm(size_t M, size_t N, size_t K, int group, const uint16_t* scales, const uint32_t* qzeros,
-                         int y_f32, int splits) {
+                         int y_f32, int glu) {
     if (M < (y_f32 ? SNX_W4_GEMM_MIN_M : SNX_W4_GEMM_MIN_M_BF16) || ((uintptr_t)scales & 3u) != 0 ||
         ((uintptr_t)qzeros & 3u) != 0 || !snx_w4a16_gemm_ok(M, N, K, group) ||
         (M < SNX_W4_GEMM_MIN_M && w4_prep_bytes(M, K) > SNEPPX_NOALLOC_SCRATCH_BYTES))
         return 0;
     return !snx_w4a16_batch_ok(M, N, K, group, scales, qzeros) ||
-           10 * snx_w4a16_gemm_cost(M, N, K, splits) <= 11 * snx_w4a16_batch_cost(M, N, K);
+           10 * snx_w4a16_gemm_cost(M, N, K, glu ? 1 : snx_w4a16_gemm_splits(M, N, K)) <= 11 * snx_w4a16_batch_cost(M, N, K);
 }
 
 /* One row, and M <= 4 within the LDS-staged small-M kernel (groups of 256 and
@@ -234,8 +234,7 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
     /* the allocation-free entry point's limit is the one its header gives, also
      * where the batch kernel would need less */
     if (noalloc && aligned && !snx_noalloc_scratch(w4_noalloc_bytes(M, N, K, group, scales, qzeros), who)) return -1;
-    if (aligned && w4_takes_gemm(M, N, K, group, scales, qzeros, y_f32,
-                                 snx_w4a16_gemm_splits(M, N, K))) {
+    if (aligned && w4_takes_gemm(M, N, K, group, scales, qzeros, y_f32, 0)) {
         /* prefill GEMM: activations prepared once into the call's scratch */
         const size_t Mp = snx_w4_prep_rows(M);
         const size_t xp_bytes = (M * K * sizeof(uint16_t) + 255) & ~(size_t)255;
@@ -446,8 +445,7 @@ int SNEPPX_qlinear_w4a16_mlp(const uint16_t* x, const uint32_t* gu_qweight, cons
     snx_clear_error();
     if (aligned16(x) && aligned16(gu_qweight) && aligned16(dn_qweight) && F % 128 == 0 &&
         w4_takes_gemm(M, 2 * F, H, group, gu_scales, gu_qzeros, 0, 1) &&
-        w4_takes_gemm(M, N, F, group, dn_scales, dn_qzeros, y_dtype == SNEPPX_FLOAT32,
-                      snx_w4a16_gemm_splits(M, N, F))) {
+        w4_takes_gemm(M, N, F, group, dn_scales, dn_qzeros, y_dtype == SNEPPX_FLOAT32, 0)) {
         /* x prepared once; the gate/up GEMM's SwiGLU epilogue writes the down
          * GEMM's prepared input (slot order + step sums) */
         const size_t Mp = snx_w4_prep_rows(M);
