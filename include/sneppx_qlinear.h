@@ -130,7 +130,8 @@ int SNEPPX_qlinear_w4a16(const uint16_t* x, const uint32_t* qweight, const uint1
  * e.g. the Llama-3-8B QKV projection at 1849 tokens), this one runs that
  * GEMM whole-K, the same
  * product with another fp32 summation order, so a bf16 output can differ
- * in its last bit.  The scratch the split-K decode and the prefill
+ * in its last bit; and a call recorded into a graph takes the batch kernel
+ * here, and kernels without scratch there.  The scratch the split-K decode and the prefill
  * GEMM need (fp32 partials, prepared activations) comes from one static
  * device array of SNEPPX_NOALLOC_SCRATCH_BYTES per GPU, held from the first
  * call on that GPU until the process ends, instead of a workspace.  A call
@@ -138,7 +139,8 @@ int SNEPPX_qlinear_w4a16(const uint16_t* x, const uint32_t* qweight, const uint1
  * example split-K partials K/1024 * M * N * 4 bytes, prefill 2 M K bytes and
  * more).  Every call on a GPU shares its array: calls that overlap on one GPU
  * (two streams, two threads) race on it and must be serialised by the
- * caller.  Nothing in the array needs to start at zero. */
+ * caller; beside it lie arrival counters that every call leaves at zero, which
+ * an overlap can leave otherwise.  Nothing in the array needs to start at zero. */
 #define SNEPPX_NOALLOC_SCRATCH_BYTES (32u << 20)
 int SNEPPX_qlinear_w4a16_noalloc(const uint16_t* x, const uint32_t* qweight,
                                  const uint16_t* scales, const uint32_t* qzeros,

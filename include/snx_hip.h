@@ -43,7 +43,11 @@ int snx_hip_device_info(char* arch, size_t arch_len, int* cu_count, int* clock_k
  * capture mode, so other threads' work is unaffected), and end returns an
  * executable graph that graph_launch replays on a stream with one host call.
  * The decode GEMVs take no workspace and record only kernel nodes (no
- * memsets).  Entry points that allocate a workspace the first time they see
+ * memsets).  A recorded call does not take the batch kernels (W4A16, W8, W8A8
+ * and MX with few rows), whose scratch it would share with other calls: it
+ * runs the kernels without one, so its result can differ from an eager call's
+ * in the rounding.  SNEPPX_qlinear_w4a16_noalloc, whose scratch is static, is
+ * the form to record for decode batches.  Entry points that allocate a workspace the first time they see
  * a shape must have run once on that stream before capture, so that the
  * workspace exists and the capture records kernels only. */
 int snx_hip_stream_begin_capture(void* stream);

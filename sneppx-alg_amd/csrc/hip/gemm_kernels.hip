@@ -1331,7 +1331,7 @@ int snx_k_i8_gemm(const int8_t* A, const int8_t* W, const float* sA, const float
         return -1;
     }
     const bool tiled = K % TBK == 0 && M >= 128 && N >= 128;
-    if (!c_i32 && (tiled ? snx_q8_batch_better(0, M, N, K) : snx_q8_batch_ok(0, M, N, K)))
+    if (!c_i32 && (tiled ? snx_q8_batch_better(0, M, N, K) : snx_q8_batch_ok(0, M, N, K)) && !snx_stream_capturing(st))
         return snx_k_q8_batch(0, A, sA, W, sW, out_bf16, bias, 0, M, N, K, st);
     if (tiled) {
         // the persistent kernel addresses operands with 31-bit buffer offsets
@@ -1386,7 +1386,7 @@ int snx_k_mx8_gemm(const uint8_t* A, const int8_t* sA, const uint8_t* W, const i
         snx_set_error("mx gemm: K %% 128 == 0 and operands below 4 GiB are required");
         return -1;
     }
-    if (snx_q8_batch_better(2 + mf, M, N, K))
+    if (snx_q8_batch_better(2 + mf, M, N, K) && !snx_stream_capturing(st))
         return snx_k_q8_batch(2 + mf, A, sA, W, sW, out, nullptr, y_f32, M, N, K, st);
     const int m = (int)M, n = (int)N, k = (int)K;
 #define SNX_MX8(F, B)                                                                       \
@@ -1408,7 +1408,7 @@ int snx_k_fp8_gemm(const uint8_t* A, const uint8_t* W, const float* sA, const fl
         return -1;
     }
     const bool tiled = K % TBK == 0 && M >= 128 && N >= 128;
-    if (tiled ? snx_q8_batch_better(1, M, N, K) : snx_q8_batch_ok(1, M, N, K))
+    if ((tiled ? snx_q8_batch_better(1, M, N, K) : snx_q8_batch_ok(1, M, N, K)) && !snx_stream_capturing(st))
         return snx_k_q8_batch(1, A, sA, W, sW, out_bf16, bias, 0, M, N, K, st);
     if (tiled) {
         const int8_t* a8 = reinterpret_cast<const int8_t*>(A);

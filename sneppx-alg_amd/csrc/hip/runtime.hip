@@ -136,6 +136,22 @@ void* snx_workspace(size_t bytes, int slot, void* stream) { return workspace(byt
 // split GEMM's arrival counters).
 void* snx_workspace_zeroed(size_t bytes, int slot, void* stream) { return workspace(bytes, slot, stream, true); }
 
+// 1 while `stream` is being captured into a graph.  A graph outlives the call
+// and may be replayed on any stream, next to other graphs and eager calls, and
+// a workspace it was recorded with may since have been replaced by a larger
+// one; so a kernel that takes a workspace is not chosen for a recorded call
+// where one without does the same.  (The legacy default stream cannot be
+// captured, and asking about it while another stream is records an error.)
+int snx_stream_capturing(void* stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (!stream) return 0;
+    if (hipStreamIsCapturing(S(stream), &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // Frees (stream-ordered) this thread's workspaces on `stream` and those that
 // ended threads left on it, for a caller about to destroy that stream.
 void snx_release_workspaces(void* stream) { snx_ws::release_stream(stream); }

@@ -130,7 +130,7 @@ int SNEPPX_qlinear_mxfp4_gemm(const uint8_t* A, const int8_t* sA, const uint8_t*
     snx_clear_error();
     const int words = ((uintptr_t)sA & 3u) == 0 && ((uintptr_t)sW & 3u) == 0;   /* exponents read as words */
     const int tiled = words && K % 256 == 0 && M >= 128 && N >= 128;
-    if (words && (tiled ? snx_q8_batch_better(6, M, N, K) : snx_q8_batch_ok(6, M, N, K)))
+    if (words && (tiled ? snx_q8_batch_better(6, M, N, K) : snx_q8_batch_ok(6, M, N, K)) && !snx_stream_capturing(stream))
         return snx_k_q8_batch(6, A, sA, W, sW, out, NULL, out_dtype == SNEPPX_FLOAT32, M, N, K, stream);
     if (tiled)
         return snx_k_mxfp4_gemm_tiled(A, sA, W, sW, out, out_dtype == SNEPPX_FLOAT32, M, N, K, stream);

@@ -116,7 +116,7 @@ int SNEPPX_qlinear_w8_gemv(const float* x, const int8_t* qweight, const float* s
     REQUIRE(K % 16 != 0 || (aligned16(x) && aligned16(qweight)),
             "qlinear_w8_gemv: x and qweight must be 16-byte aligned");
     snx_clear_error();
-    if (snx_w8_batch_ok(M, N, K, qweight)) {
+    if (snx_w8_batch_ok(M, N, K, qweight) && !snx_stream_capturing(stream)) {
         const int splits = snx_w8_batch_splits(M, N, K);
         void* xp = snx_workspace(snx_w8_batch_xp_bytes(M, K), 1, stream);
         void* part = NULL;
@@ -167,14 +167,15 @@ static size_t w4_prep_bytes(size_t M, size_t K) {
  * split K): where it may and the batch kernel is not estimated to be faster by a
  * tenth (what the estimates are off by).
  * Below SNX_W4_GEMM_MIN_M only where the allocation-free entry point, which
- * decides alike, has the scratch for it. */
+ * decides alike, has the scratch for it.  recorded: the call is captured into
+ * a graph and neither the batch kernel nor a smaller GEMM is a choice. */
 static int w4_takes_gemm(size_t M, size_t N, size_t K, int group, const uint16_t* scales, const uint32_t* qzeros,
-                         int y_f32, int glu) {
-    if (M < (y_f32 ? SNX_W4_GEMM_MIN_M : SNX_W4_GEMM_MIN_M_BF16) || ((uintptr_t)scales & 3u) != 0 ||
+                         int y_f32, int glu, int recorded) {
+    if (M < (y_f32 || recorded ? SNX_W4_GEMM_MIN_M : SNX_W4_GEMM_MIN_M_BF16) || ((uintptr_t)scales & 3u) != 0 ||
         ((uintptr_t)qzeros & 3u) != 0 || !snx_w4a16_gemm_ok(M, N, K, group) ||
         (M < SNX_W4_GEMM_MIN_M && w4_prep_bytes(M, K) > SNEPPX_NOALLOC_SCRATCH_BYTES))
         return 0;
-    return !snx_w4a16_batch_ok(M, N, K, group, scales, qzeros) ||
+    return recorded || !snx_w4a16_batch_ok(M, N, K, group, scales, qzeros) ||
            10 * snx_w4a16_gemm_cost(M, N, K, glu ? 1 : snx_w4a16_gemm_splits(M, N, K)) <= 11 * snx_w4a16_batch_cost(M, N, K);
 }
 
@@ -234,7 +235,9 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
     /* the allocation-free entry point's limit is the one its header gives, also
      * where the batch kernel would need less */
     if (noalloc && aligned && !snx_noalloc_scratch(w4_noalloc_bytes(M, N, K, group, scales, qzeros), who)) return -1;
-    if (aligned && w4_takes_gemm(M, N, K, group, scales, qzeros, y_f32, 0)) {
+    /* (a call of the M = 1 kernels takes no workspace, and is not asked about) */
+    const int recorded = !noalloc && !(M == 1 && w4_small(M, K, group, scales, qzeros)) && snx_stream_capturing(stream);
+    if (aligned && w4_takes_gemm(M, N, K, group, scales, qzeros, y_f32, 0, recorded)) {
         /* prefill GEMM: activations prepared once into the call's scratch */
         const size_t Mp = snx_w4_prep_rows(M);
         const size_t xp_bytes = (M * K * sizeof(uint16_t) + 255) & ~(size_t)255;
@@ -262,7 +265,7 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
         /* 2 <= M <= 16: one persistent workgroup per CU, activations staged once */
         return snx_k_w4a16_gemv_mt(x, qweight, scales, qzeros, NULL, y, bias, y_f32, M, N, K, stream);
     }
-    if (aligned && !w4_small(M, K, group, scales, qzeros) && !w4_short(M, N, K, group) &&
+    if (aligned && !recorded && !w4_small(M, K, group, scales, qzeros) && !w4_short(M, N, K, group) &&
         snx_w4a16_batch_ok(M, N, K, group, scales, qzeros))
         return w4_batch(who, noalloc, x, qweight, scales, qzeros, bias, y, y_f32, M, N, K, group, 0, stream);
     const int kspan = snx_w4a16_splitk_span(M, K, group);
@@ -396,7 +399,8 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
     REQUIRE(aligned16(out), "qlinear_w4a16_swiglu: out must be 16-byte aligned");
     snx_clear_error();
     const int aligned = aligned16(x) && aligned16(qweight);
-    if (aligned && w4_takes_gemm(M, 2 * F, K, group, scales, qzeros, 0, 1)) {
+    const int recorded = snx_stream_capturing(stream);
+    if (aligned && w4_takes_gemm(M, 2 * F, K, group, scales, qzeros, 0, 1, recorded)) {
         const size_t Mp = snx_w4_prep_rows(M);
         const size_t xp_bytes = (M * K * sizeof(uint16_t) + 255) & ~(size_t)255;
         char* ws = (char*)snx_workspace(w4_prep_bytes(M, K), 1, stream);
@@ -414,7 +418,7 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
         return snx_k_w4a16_gemv1_swiglu(x, qweight, scales, qzeros, bias, out, F, K, group, stream);
     /* (up to 8 rows of the persistent decode kernel's shapes its fp32 rows and
      * the rule's own pass stay faster: 20.8 against 22.5 us at F = 14336) */
-    if (aligned && !(M <= 8 && snx_w4a16_mt_ok(M, K, group, 0)) && !(M == 1 && w4_small(M, K, group, scales, qzeros)) &&
+    if (aligned && !recorded && !(M <= 8 && snx_w4a16_mt_ok(M, K, group, 0)) && !(M == 1 && w4_small(M, K, group, scales, qzeros)) &&
         !w4_short(M, 2 * F, K, group) &&
         snx_w4a16_batch_ok(M, 2 * F, K, group, scales, qzeros))
         return w4_batch("qlinear_w4a16_swiglu", 0, x, qweight, scales, qzeros, bias, out, 0, M, F, K, group, 1, stream);
@@ -443,9 +447,10 @@ int SNEPPX_qlinear_w4a16_mlp(const uint16_t* x, const uint32_t* gu_qweight, cons
     REQUIRE(y_dtype == SNEPPX_BFLOAT16 || y_dtype == SNEPPX_FLOAT32,
             "qlinear_w4a16_mlp: y_dtype must be SNEPPX_BFLOAT16 or SNEPPX_FLOAT32");
     snx_clear_error();
+    const int recorded = snx_stream_capturing(stream);
     if (aligned16(x) && aligned16(gu_qweight) && aligned16(dn_qweight) && F % 128 == 0 &&
-        w4_takes_gemm(M, 2 * F, H, group, gu_scales, gu_qzeros, 0, 1) &&
-        w4_takes_gemm(M, N, F, group, dn_scales, dn_qzeros, y_dtype == SNEPPX_FLOAT32, 0)) {
+        w4_takes_gemm(M, 2 * F, H, group, gu_scales, gu_qzeros, 0, 1, recorded) &&
+        w4_takes_gemm(M, N, F, group, dn_scales, dn_qzeros, y_dtype == SNEPPX_FLOAT32, 0, recorded)) {
         /* x prepared once; the gate/up GEMM's SwiGLU epilogue writes the down
          * GEMM's prepared input (slot order + step sums) */
         const size_t Mp = snx_w4_prep_rows(M);

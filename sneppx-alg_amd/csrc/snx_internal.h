@@ -26,6 +26,10 @@ void* snx_workspace_zeroed(size_t bytes, int slot, void* stream);
 void snx_release_workspaces(void* stream);
 /* workspaces held now, by live threads and left by ended ones (for tests) */
 long snx_workspace_count(void);
+/* 1 while `stream` is being captured: the batch kernels, whose scratch would
+ * be shared with other calls and replays, are not chosen then (the
+ * allocation-free entry point, which documents that sharing, takes them) */
+int snx_stream_capturing(void* stream);
 /* the current device's static scratch array (noalloc.hip) when `bytes` fit
  * in it, else NULL with the error text set (prefixed by `who`) */
 void* snx_noalloc_scratch(size_t bytes, const char* who);
