@@ -459,6 +459,48 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
         for (int o = 0; o < OWN; o++) up[o] = red[(2 * NP + kw + o * KW) * 64];
     }
 
+    // Groups below 128: an infinite activation (or one past 1e37) makes both
+    // products infinite and their difference NaN where sum x (q - z) s is an
+    // infinity or a number.  Such results are computed once more, in that form,
+    // by their own lane.  Costs calls without them their test and the code:
+    // N = 6144, K = 4096, groups of 64: M = 16 10.6 -> 10.7 us, 96 18.3 -> 20.0
+    // (k_w4a16_generic, which these groups ran before, 460 us at M = 16).
+    // Wider groups came from kernels that subtract 128 + z likewise.
+    if constexpr (GS < 128) {
+        auto finite = [](float f) { return (__builtin_bit_cast(uint32_t, f) & 0x7F800000u) != 0x7F800000u; };
+        bool fine = true;
+#pragma unroll
+        for (int o = 0; o < OWN; o++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) fine = fine && finite(res[o][e]) && finite(up[o][e]);
+        if (__builtin_expect(__ballot(!fine) != 0, 0)) {
+#pragma unroll 1
+            for (int it = 0; it < (glu ? 2 : 1) * OWN * 4; it++) {
+                const int half = it >= OWN * 4, at = it - half * OWN * 4, p = kw + (at >> 2) * KW;
+                const int s = p % NS, i = (p / NS) % MT, v = p / (NS * MT);
+                const int n = c0 + s * MR + r, m = m0 + i * MR + (MR == 32 ? 8 * v + 4 * q : 4 * q) + (at & 3);
+                const size_t row = (size_t)(n < N ? n : N - 1) + (half ? (size_t)N : 0), mc = m < M ? m : M - 1;
+                float f = 0.0f;
+#pragma unroll 1
+                for (int w = 0; w < K / 8; w++) {
+                    const uint32_t g = (uint32_t)(w * 8) >> gshift, word = qw[row * (K / 8) + w];
+                    const int z = qz ? (int)((qz[row * ZW + (g >> 3)] >> (4 * (g & 7))) & 15u) : 8;
+                    const float scale = f16_dev(scales[row * G + g]);
+#pragma unroll 1
+                    for (int t = 0; t < 8; t++)
+                        f += bf16_to_f32(x[mc * K + w * 8 + t]) * ((float)((int)((word >> (4 * t)) & 15u) - z) * scale);
+                }
+#pragma unroll
+                for (int o = 0; o < OWN; o++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        if (it == o * 4 + e && !finite(res[o][e])) res[o][e] = f;
+                        if (it == (OWN + o) * 4 + e && !finite(up[o][e])) up[o][e] = f;
+                    }
+            }
+        }
+    }
+
     // rows past M lie past the buffer's records and are dropped there; lanes
     // of columns past N take an offset that is
     const uint32_t eb = y_f32 ? 4 : 2;

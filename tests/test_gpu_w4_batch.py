@@ -97,3 +97,27 @@ def test_w4_batch_swiglu_matches_float64(lib, oracle, M, F, K, group, zeros, bia
     torch.cuda.synchronize()
     err = rel_err(got.float().cpu().numpy(), want)
     assert err <= TOL_BF16
+
+
+@pytest.mark.parametrize("M,N,K,group", [(6, 70, 512, 64), (16, 40, 2048, 32), (40, 130, 512, 32), (96, 100, 2048, 64)])
+def test_w4_batch_small_groups_with_extreme_activations(lib, oracle, M, N, K, group):
+    """Infinities, NaN and activations whose product with a bare code overflows: the
+    result of sum x (q - z) s.  Terms are added one after the other: K roundings of
+    2^-24 of the sum of their sizes."""
+    print(f"[gpu] w4 batch extreme activations M={M} N={N} K={K} g={group}", flush=True)
+    (qw, sc, qz), v = _case(oracle, N, K, group, True, M + group)
+    x = bf16_to_f32(bf16_bits(np.random.default_rng(M).normal(0.3, 1, (M, K)).astype(np.float32)))
+    x[1, 7], x[2, K - 1], x[3, 40], x[4, 9] = np.inf, -np.inf, np.nan, 2.0**127
+    y = torch.full((M, N), 7.0, device=DEV)
+    lib.qlinear_w4a16(to_dev(x).to(torch.bfloat16), qw, sc, qz, None, K // group, y, group)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ v.T
+    assert np.isinf(want[1]).any() and np.isfinite(want[4]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want))
+    assert np.array_equal(np.sign(got[np.isinf(got)]), np.sign(want[np.isinf(want)]))
+    rows = np.isfinite(x).all(axis=1)
+    size = np.abs(x[rows]).astype(np.float64) @ np.abs(v).T
+    assert float((np.abs(got[rows] - want[rows]) / size).max()) <= K * 2.0**-24
