@@ -44,12 +44,18 @@ int snx_hip_device_info(char* arch, size_t arch_len, int* cu_count, int* clock_k
  * executable graph that graph_launch replays on a stream with one host call.
  * The decode GEMVs take no workspace and record only kernel nodes (no
  * memsets).  A recorded call does not take the batch kernels (W4A16, W8, W8A8
- * and MX with few rows), whose scratch it would share with other calls: it
- * runs the kernels without one, so its result can differ from an eager call's
- * in the rounding.  SNEPPX_qlinear_w4a16_noalloc, whose scratch is static, is
- * the form to record for decode batches.  Entry points that allocate a workspace the first time they see
- * a shape must have run once on that stream before capture, so that the
- * workspace exists and the capture records kernels only. */
+ * and MX with few rows), whose scratch it would share with other calls, but
+ * the kernels that the other shapes run; its result can differ from an eager
+ * call's in the rounding.  SNEPPX_qlinear_w4a16_noalloc, whose scratch is
+ * static, is the form to record for decode batches.
+ * A recorded call that needs a workspace all the same (W4A16 split-K decode and
+ * prefill GEMM, the fp32 rows of a SwiGLU, W8A8 GEMMs in two K spans, gathered
+ * or quantized activations) shares its stream's with the eager calls of the
+ * capturing thread: replay such a graph on that stream, or where nothing else
+ * runs there meanwhile.  The workspace need not exist before the capture (a new
+ * one is taken outside of it, so only kernels are recorded); it stays at its
+ * address for the replays, also when a later call needs a larger one, until
+ * SNEPPX_qlinear_release_workspaces(stream). */
 int snx_hip_stream_begin_capture(void* stream);
 int snx_hip_stream_end_capture(void* stream, void** graph_exec);
 int snx_hip_graph_launch(void* graph_exec, void* stream);

@@ -1272,11 +1272,11 @@ int launch_8wp(const int8_t* A, const int8_t* W, const float* sA, const float* s
     // the span partials (one 229,376-byte slot per unit and wave group) and
     // the arrival counters of the (tile, wave) pairs, which the kernel leaves at 0
     const size_t slots = (size_t)ntiles * split * 8 * (4 * TFN * 64);
-    i32x4* part = static_cast<i32x4*>(snx_workspace(slots * sizeof(i32x4), 3, st));
-    uint32_t* cnt = static_cast<uint32_t*>(snx_workspace_zeroed((size_t)ntiles * 8 * sizeof(uint32_t), 4, st));
-    if (!part || !cnt) return -1;
-    return launch_8wp_s<FP8, RAW, BIAS, 2>(A, W, sA, sW, Craw, out, bias, M, N, K, tiles_m, tiles_n, grid, part,
-                                          cnt, st);
+    void* part = nullptr;
+    uint32_t* cnt = nullptr;
+    if (snx_span_workspaces(slots * sizeof(i32x4), (size_t)ntiles * 8 * sizeof(uint32_t), st, &part, &cnt)) return -1;
+    return launch_8wp_s<FP8, RAW, BIAS, 2>(A, W, sA, sW, Craw, out, bias, M, N, K, tiles_m, tiles_n, grid,
+                                          static_cast<i32x4*>(part), cnt, st);
 }
 
 template <bool FP8, bool RAW, bool BIAS>

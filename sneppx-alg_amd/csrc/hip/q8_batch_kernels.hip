@@ -393,15 +393,14 @@ int launch(const Batch& a) {
     const int steps = (a.K + kind_step(KIND) - 1) / kind_step(KIND);
     const size_t tiles = tiles_of(a.M, a.N, 32 * MT);
     const int splits = splits_of(tiles, steps);
-    uint32_t *part = nullptr, *cnt = nullptr;
-    if (splits > 1) {
-        part = static_cast<uint32_t*>(snx_workspace(tiles * splits * (32 * MT) * BN * 4, 3, a.s));
-        cnt = static_cast<uint32_t*>(snx_workspace_zeroed(tiles * 4 * KW * sizeof(uint32_t), 4, a.s));
-        if (!part || !cnt) return -1;
-    }
+    void* part = nullptr;
+    uint32_t* cnt = nullptr;
+    if (splits > 1 && snx_span_workspaces(tiles * splits * (32 * MT) * BN * 4, tiles * 4 * KW * sizeof(uint32_t), a.s,
+                                          &part, &cnt))
+        return -1;
     const dim3 grid((a.N + BN - 1) / BN, splits, (a.M + 32 * MT - 1) / (32 * MT));
     k_q8_batch<KIND, MT, RING><<<grid, 256 * KW, bytes, a.s>>>(a.A, a.sA, a.W, a.sW, a.out, a.bias, a.y_f32, a.M, a.N,
-                                                             a.K, steps / splits, steps % splits, part, cnt);
+                                                             a.K, steps / splits, steps % splits, static_cast<uint32_t*>(part), cnt);
     return snx_launch_check("k_q8_batch");
 }
 

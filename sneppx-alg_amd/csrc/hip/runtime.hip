@@ -36,9 +36,9 @@ __global__ void __launch_bounds__(256) k_fill_zero_u32(uint32_t* __restrict__ p,
 // The library's internal scratch (split-K partials, prepared activations,
 // gathers) comes from per-thread workspaces keyed by (device, stream, slot):
 // ws_registry.h holds the rules (no sharing between threads, stream-ordered
-// growth, buffers of ended threads adopted by later ones).  Here it gets the
-// device side: the stream-ordered pool, and a fill kernel for zeroed
-// buffers.
+// growth, buffers of ended threads adopted by later ones, nothing allocated or
+// freed on a stream that is being captured).  Here it gets the device side: the
+// stream-ordered pool, and a fill kernel for zeroed buffers.
 namespace {
 void* ws_alloc(size_t bytes, void* stream, bool zeroed) {
     void* p = nullptr;
@@ -57,13 +57,43 @@ void* ws_alloc(size_t bytes, void* stream, bool zeroed) {
 
 void ws_release(void* p, void* stream) { (void)hipFreeAsync(p, S(stream)); }
 
-void* workspace(size_t bytes, int slot, void* stream, bool zeroed) {
-    static std::once_flag once;
-    std::call_once(once, [] { snx_ws::init(ws_alloc, ws_release); });
-    int dev = 0;
-    if (check(hipGetDevice(&dev), "hipGetDevice")) return nullptr;
-    return snx_ws::get(dev, stream, slot, bytes, zeroed);
+// For a recorded call: from the pool on a stream of its own, complete before
+// this returns.  A thread that captures a stream may wait for another one only
+// in the relaxed capture mode.
+void* ws_apart(size_t bytes, bool zeroed) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (check(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode")) return nullptr;
+    void *p = nullptr, *own = nullptr;
+    if (!snx_hip_stream_create(&own)) {
+        p = ws_alloc(bytes, own, zeroed);
+        if (snx_hip_stream_sync(own) && p) {
+            ws_release(p, own);
+            p = nullptr;
+        }
+        (void)snx_hip_stream_destroy(own);
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return p;
 }
+
+// The buffers of one call, which asks once whether it is being recorded.
+class Workspaces {
+public:
+    explicit Workspaces(void* stream) : stream_(stream) {
+        static std::once_flag once;
+        std::call_once(once, [] { snx_ws::init(ws_alloc, ws_release, ws_apart); });
+        ok_ = check(hipGetDevice(&dev_), "hipGetDevice") == 0;
+        recorded_ = snx_stream_capturing(stream);
+    }
+    void* get(size_t bytes, int slot, bool zeroed) const {
+        return ok_ ? snx_ws::get(dev_, stream_, slot, bytes, zeroed, recorded_) : nullptr;
+    }
+
+private:
+    void* stream_;
+    int dev_ = 0;
+    bool ok_, recorded_;
+};
 }  // namespace
 
 extern "C" {
@@ -129,19 +159,25 @@ int snx_hip_free_async(void* ptr, void* stream) {
     return ptr ? check(hipFreeAsync(ptr, S(stream)), "hipFreeAsync") : 0;
 }
 
-void* snx_workspace(size_t bytes, int slot, void* stream) { return workspace(bytes, slot, stream, false); }
+void* snx_workspace(size_t bytes, int slot, void* stream) { return Workspaces(stream).get(bytes, slot, false); }
 
-// As snx_workspace, with a new buffer zero-filled (stream-ordered) when it is
-// taken; for data the caller's kernels return to zero before they end (the
-// split GEMM's arrival counters).
-void* snx_workspace_zeroed(size_t bytes, int slot, void* stream) { return workspace(bytes, slot, stream, true); }
+// Slots 3 and 4.  A new buffer of counters is zero-filled (stream-ordered) when
+// it is taken; the kernels that count in it return it to zero before they end.
+int snx_span_workspaces(size_t part_bytes, size_t cnt_bytes, void* stream, void** part, uint32_t** cnt) {
+    const Workspaces ws(stream);
+    *part = ws.get(part_bytes, 3, false);
+    *cnt = *part ? static_cast<uint32_t*>(ws.get(cnt_bytes, 4, true)) : nullptr;
+    return *cnt ? 0 : -1;
+}
 
 // 1 while `stream` is being captured into a graph.  A graph outlives the call
-// and may be replayed on any stream, next to other graphs and eager calls, and
-// a workspace it was recorded with may since have been replaced by a larger
-// one; so a kernel that takes a workspace is not chosen for a recorded call
-// where one without does the same.  (The legacy default stream cannot be
-// captured, and asking about it while another stream is records an error.)
+// and may be replayed on any stream, next to other graphs and eager calls that
+// would share a workspace with it; so the batch kernels, which take one where
+// the kernels they replace do not, are not chosen for a recorded call.  What it
+// runs instead may take a workspace of the stream all the same (split-K, the
+// fp32 rows of a SwiGLU, the prefill GEMM, the W8A8 spans).  (The legacy default
+// stream cannot be captured, and asking about it while another stream is
+// records an error.)
 int snx_stream_capturing(void* stream) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (!stream) return 0;

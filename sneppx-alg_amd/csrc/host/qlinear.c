@@ -122,11 +122,9 @@ int SNEPPX_qlinear_w8_gemv(const float* x, const int8_t* qweight, const float* s
         void* part = NULL;
         uint32_t* cnt = NULL;
         if (!xp) return -1;
-        if (splits > 1) {
-            part = snx_workspace(snx_w8_batch_part_bytes(M, N, splits), 3, stream);
-            cnt = (uint32_t*)snx_workspace_zeroed(snx_w8_batch_cnt_bytes(M, N), 4, stream);
-            if (!part || !cnt) return -1;
-        }
+        if (splits > 1 && snx_span_workspaces(snx_w8_batch_part_bytes(M, N, splits), snx_w8_batch_cnt_bytes(M, N),
+                                              stream, &part, &cnt))
+            return -1;
         return snx_k_w8_batch(x, qweight, scales, y, bias, M, N, K, splits, xp, part, cnt, stream);
     }
     return snx_k_w8_gemv(x, qweight, scales, y, bias, M, N, K, stream);
@@ -150,9 +148,13 @@ static int w4_batch(const char* who, int noalloc, const uint16_t* x, const uint3
     uint32_t* cnt = NULL;
     if (splits > 1) {
         const size_t pb = snx_w4a16_batch_part_bytes(M, rows, splits), cb = snx_w4a16_batch_cnt_bytes(M, rows);
-        part = noalloc ? snx_noalloc_scratch(pb, who) : snx_workspace(pb, 3, stream);
-        cnt = (uint32_t*)(noalloc ? snx_noalloc_counters(cb, who) : snx_workspace_zeroed(cb, 4, stream));
-        if (!part || !cnt) return -1;
+        if (!noalloc) {
+            if (snx_span_workspaces(pb, cb, stream, &part, &cnt)) return -1;
+        } else {
+            part = snx_noalloc_scratch(pb, who);
+            cnt = (uint32_t*)snx_noalloc_counters(cb, who);
+            if (!part || !cnt) return -1;
+        }
     }
     return snx_k_w4a16_batch(x, qweight, scales, qzeros, y, bias, y_f32, M, N, K, group, glu, splits, part, cnt,
                              stream);
@@ -250,11 +252,9 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
         const int splits = noalloc ? 1 : snx_w4a16_gemm_splits(M, N, K);
         void* part = NULL;
         uint32_t* cnt = NULL;
-        if (splits > 1) {
-            part = snx_workspace(snx_w4a16_gemm_part_bytes(M, N, splits), 3, stream);
-            cnt = (uint32_t*)snx_workspace_zeroed(snx_w4a16_gemm_cnt_bytes(M, N), 4, stream);
-            if (!part || !cnt) return -1;
-        }
+        if (splits > 1 && snx_span_workspaces(snx_w4a16_gemm_part_bytes(M, N, splits), snx_w4a16_gemm_cnt_bytes(M, N),
+                                              stream, &part, &cnt))
+            return -1;
         int rc = snx_k_w4_prep_x(x, xp, xs, M, K, Mp, stream);
         if (!rc) rc = snx_k_w4a16_gemm(xp, xs, qweight, scales, qzeros, y, bias, y_f32, M, N, K,
                                        group, Mp, splits, part, cnt, stream);
@@ -466,11 +466,9 @@ int SNEPPX_qlinear_w4a16_mlp(const uint16_t* x, const uint32_t* gu_qweight, cons
         const int splits = snx_w4a16_gemm_splits(M, N, F);
         void* part = NULL;
         uint32_t* cnt = NULL;
-        if (splits > 1) {
-            part = snx_workspace(snx_w4a16_gemm_part_bytes(M, N, splits), 3, stream);
-            cnt = (uint32_t*)snx_workspace_zeroed(snx_w4a16_gemm_cnt_bytes(M, N), 4, stream);
-            if (!part || !cnt) return -1;
-        }
+        if (splits > 1 && snx_span_workspaces(snx_w4a16_gemm_part_bytes(M, N, splits), snx_w4a16_gemm_cnt_bytes(M, N),
+                                              stream, &part, &cnt))
+            return -1;
         int rc = snx_k_w4_prep_x(x, xp, xs, M, H, Mp, stream);
         if (!rc) rc = snx_k_w4a16_gemm_swiglu_prep(xp, xs, gu_qweight, gu_scales, gu_qzeros, ap, as, gu_bias,
                                                    M, F, H, group, Mp, stream);

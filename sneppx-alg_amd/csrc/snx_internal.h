@@ -19,16 +19,17 @@ void snx_set_error(const char* fmt, ...);
  * the calling host thread; slot 1 is for a call made from inside another
  * one.  NULL on failure. */
 void* snx_workspace(size_t bytes, int slot, void* stream);
-/* as snx_workspace; a newly taken buffer is zero-filled on `stream` first */
-void* snx_workspace_zeroed(size_t bytes, int slot, void* stream);
+/* the partials of K spans and their arrival counters, which are zero and left
+ * zero by every call; 0, or -1 with the error text set */
+int snx_span_workspaces(size_t part_bytes, size_t cnt_bytes, void* stream, void** part, uint32_t** cnt);
 /* stream-ordered release of the calling thread's workspaces on `stream` and
  * of those that ended threads left on it */
 void snx_release_workspaces(void* stream);
 /* workspaces held now, by live threads and left by ended ones (for tests) */
 long snx_workspace_count(void);
-/* 1 while `stream` is being captured: the batch kernels, whose scratch would
- * be shared with other calls and replays, are not chosen then (the
- * allocation-free entry point, which documents that sharing, takes them) */
+/* 1 while `stream` is being captured: the batch kernels are not chosen then
+ * (the allocation-free entry point, which documents that its scratch is shared,
+ * takes them) */
 int snx_stream_capturing(void* stream);
 /* the current device's static scratch array (noalloc.hip) when `bytes` fit
  * in it, else NULL with the error text set (prefixed by `who`) */

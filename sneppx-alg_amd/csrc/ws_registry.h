@@ -2,7 +2,7 @@
 // (device, stream, slot) for each host thread, with no device calls of its
 // own: allocation and stream-ordered release go through the two callbacks
 // given to snx_ws::init (HIP's stream-ordered pool in runtime.hip, malloc in
-// the CPU test of this logic).
+// the CPU tests of this logic).
 //
 // Rules:
 //  * A thread looks its buffers up in a thread_local table (a few entries:
@@ -20,6 +20,15 @@
 //    ended, so work queued there afterwards is ordered behind it.  A pool of
 //    short-lived request threads therefore holds as many buffers per
 //    (stream, slot) as it has threads alive at once, not as it ever had.
+//  * While a stream is captured into a graph, nothing may be allocated or freed
+//    on it: that would become a part of the graph (memory that the graph owns, a
+//    fill that runs at replays only, a free at every replay).  A recorded call's
+//    new buffer is allocated and zeroed apart, complete when get() returns, and
+//    serves the stream's eager calls too.
+//  * A buffer that a recorded call has taken is kept at its address for the
+//    replays: where a larger request takes a new one, the old one stays (not
+//    handed out any more) until release_stream.  Sizes grow by a quarter or
+//    more, so those that stay are less than four times the largest.
 //  * release_stream(stream) frees the calling thread's buffers and every
 //    orphan on `stream`, for a caller about to destroy that stream.
 #ifndef SNX_WS_REGISTRY_H
@@ -35,19 +44,25 @@ namespace snx_ws {
 // alloc: a buffer of `bytes` usable by work queued on `stream` (zero-filled
 // on `stream` when `zeroed`), nullptr on failure.  release: frees `p` after
 // the work already queued on `stream`.
+// apart: a buffer usable anywhere at once, taken without touching any stream
+// that is being captured; release() frees it too.
 using AllocFn = void* (*)(size_t bytes, void* stream, bool zeroed);
 using ReleaseFn = void (*)(void* p, void* stream);
+using ApartFn = void* (*)(size_t bytes, bool zeroed);
 
 struct Buf {
     int dev, slot;
     void* stream;
     void* ptr;
     size_t bytes;
+    bool recorded;                 // a graph may use it
+    bool replaced;                 // by a larger one: kept for the graph alone
 };
 
 struct Shared {
     AllocFn alloc = nullptr;
     ReleaseFn release = nullptr;
+    ApartFn apart = nullptr;
     std::mutex mu;                 // guards orphans
     std::vector<Buf> orphans;
     std::atomic<long> live{0};     // buffers held by threads and orphans
@@ -73,27 +88,29 @@ inline Table& table() {
     return t;
 }
 
-inline void init(AllocFn alloc, ReleaseFn release) {
+inline void init(AllocFn alloc, ReleaseFn release, ApartFn apart = nullptr) {
     Shared& s = shared();
     s.alloc = alloc;
     s.release = release;
+    s.apart = apart;
 }
 
-// A buffer of at least `bytes` for this thread's work on (dev, stream, slot).
-inline void* get(int dev, void* stream, int slot, size_t bytes, bool zeroed) {
+// A buffer of at least `bytes` for this thread's work on (dev, stream, slot);
+// recorded: `stream` is being captured.
+inline void* get(int dev, void* stream, int slot, size_t bytes, bool zeroed, bool recorded = false) {
     Shared& s = shared();
     Table& t = table();
     if (bytes == 0) bytes = 1;
     Buf* b = nullptr;
     for (auto& e : t.bufs)
-        if (e.dev == dev && e.slot == slot && e.stream == stream) { b = &e; break; }
+        if (!e.replaced && e.dev == dev && e.slot == slot && e.stream == stream) { b = &e; break; }
     if (!b) {
         // adopt the largest orphan of this key, if any
         std::lock_guard<std::mutex> lock(s.mu);
         size_t best = s.orphans.size();
         for (size_t i = 0; i < s.orphans.size(); i++) {
             const Buf& o = s.orphans[i];
-            if (o.dev == dev && o.slot == slot && o.stream == stream &&
+            if (!o.replaced && o.dev == dev && o.slot == slot && o.stream == stream &&
                 (best == s.orphans.size() || o.bytes > s.orphans[best].bytes))
                 best = i;
         }
@@ -104,16 +121,26 @@ inline void* get(int dev, void* stream, int slot, size_t bytes, bool zeroed) {
             b = &t.bufs.back();
         }
     }
-    if (b && b->bytes >= bytes) return b->ptr;
+    if (b && b->bytes >= bytes) {
+        b->recorded |= recorded;
+        return b->ptr;
+    }
     const size_t want = (bytes + (bytes >> 2) + 4095) & ~(size_t)4095;   // +25% headroom
-    void* p = s.alloc(want, stream, zeroed);
+    const bool keep = b && (b->recorded || recorded);
+    if (!b || keep) {
+        const size_t at = b ? (size_t)(b - t.bufs.data()) : 0;
+        t.bufs.reserve(t.bufs.size() + 1);   // before the allocation: this may throw
+        if (b) b = &t.bufs[at];
+    }
+    void* p = recorded ? s.apart(want, zeroed) : s.alloc(want, stream, zeroed);
     if (!p) return nullptr;
-    if (b) {
+    if (b && !keep) {
         s.release(b->ptr, stream);
         b->ptr = p;
         b->bytes = want;
     } else {
-        t.bufs.push_back(Buf{dev, slot, stream, p, want});
+        if (b) b->replaced = true;
+        t.bufs.push_back(Buf{dev, slot, stream, p, want, recorded, false});
         s.live.fetch_add(1, std::memory_order_relaxed);
     }
     return p;
