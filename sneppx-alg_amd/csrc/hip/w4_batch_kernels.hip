@@ -459,79 +459,150 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
         for (int o = 0; o < OWN; o++) up[o] = red[(2 * NP + kw + o * KW) * 64];
     }
 
-    // Groups below 128: an infinite activation (or one past 1e37) makes both
-    // products infinite and their difference NaN where sum x (q - z) s is an
-    // infinity or a number.  Such results are computed once more, in that form,
-    // by their own lane.  Costs calls without them their test and the code:
-    // N = 6144, K = 4096, groups of 64: M = 16 10.6 -> 10.7 us, 96 18.3 -> 20.0
-    // (k_w4a16_generic, which these groups ran before, 460 us at M = 16).
-    // Wider groups came from kernels that subtract 128 + z likewise.
-    if constexpr (GS < 128) {
-        auto finite = [](float f) { return (__builtin_bit_cast(uint32_t, f) & 0x7F800000u) != 0x7F800000u; };
-        bool fine = true;
+    // rows past M lie past the buffer's records and are dropped there; lanes
+    // of columns past N take an offset that is
+    auto finish = [&] {
+        const uint32_t eb = y_f32 ? 4 : 2;
+        const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(y, (short)0, (int)((uint32_t)M * (uint32_t)N * eb), 0x00020000);
+#pragma unroll
+        for (int o = 0; o < OWN; o++) {
+            const int p = kw + o * KW;
+            const int s = p % NS, i = (p / NS) % MT, v = p / (NS * MT);
+            const int n = c0 + s * MR + r, m = m0 + i * MR + (MR == 32 ? 8 * v + 4 * q : 4 * q);
+            uint32_t off = n < N ? ((uint32_t)m * (uint32_t)N + (uint32_t)n) * eb : 0x80000000u;
+            if (bias) res[o] += bias[n < N ? n : N - 1];
+            if (glu) {
+                if (bias) up[o] += bias[N + (n < N ? n : N - 1)];
+#pragma unroll
+                for (int e = 0; e < 4; e++) res[o][e] = silu_mul_fast(res[o][e], up[o][e]);
+            }
+            if (y_f32) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float f = res[o][e];
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), ry, off, 0, 0);
+                    off += (uint32_t)N * 4u;
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    __builtin_amdgcn_raw_buffer_store_b16(bf16_out(res[o][e]), ry, off, 0, 0);
+                    off += (uint32_t)N * 2u;
+                }
+            }
+        }
+    };
+
+    // Groups below 128: an infinite activation (or one past 1e37) makes both products infinite and
+    // their difference NaN where sum x (q - z) s is an infinity or a number.  A
+    // wave with a result that is not finite computes its columns once more in
+    // that form, straight from memory, and takes from it what was not finite:
+    // codes as bf16 (q - z) 2^-16, whose products with any activation are finite,
+    // 32 rows at a time, as K / GS round trips to memory whatever the number of
+    // such results.  N = 6144, K = 4096, groups of 64, M = 96: 0.29 ms with one
+    // row of them, 0.51 with 96 (k_w4a16_generic, which these groups ran before,
+    // 2.7).  It stores its results itself: calls without such results then pay for
+    // the test alone (18.5 us at 96 rows; 18.9 where the two ways met before the
+    // stores).
+    f32x4 odd = {};                 // NaN where a result is not finite
+#pragma unroll
+    for (int o = 0; o < OWN; o++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) odd[e] = __builtin_fmaf(0.0f, res[o][e], odd[e]);
+    if (glu) {
 #pragma unroll
         for (int o = 0; o < OWN; o++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) fine = fine && finite(res[o][e]) && finite(up[o][e]);
-        if (__builtin_expect(__ballot(!fine) != 0, 0)) {
+            for (int e = 0; e < 4; e++) odd[e] = __builtin_fmaf(0.0f, up[o][e], odd[e]);
+    }
+    const float any = (odd[0] + odd[1]) + (odd[2] + odd[3]);
+    if (GS < 128 && __builtin_expect(__ballot(any != any) != 0, 0)) {
+        constexpr int RB = MR / 16;             // blocks of 16 rows, by two of 16 columns
+        const int c16 = lane & 15, q16 = lane >> 4;
 #pragma unroll 1
-            for (int it = 0; it < (glu ? 2 : 1) * OWN * 4; it++) {
-                const int half = it >= OWN * 4, at = it - half * OWN * 4, p = kw + (at >> 2) * KW;
-                const int s = p % NS, i = (p / NS) % MT, v = p / (NS * MT);
-                const int n = c0 + s * MR + r, m = m0 + i * MR + (MR == 32 ? 8 * v + 4 * q : 4 * q) + (at & 3);
-                const size_t row = (size_t)(n < N ? n : N - 1) + (half ? (size_t)N : 0), mc = m < M ? m : M - 1;
-                float f = 0.0f;
+        for (int half = 0; half <= glu; half++) {
+            size_t row[2];
+#pragma unroll
+            for (int cb = 0; cb < 2; cb++) {
+                const int n = c0 + 16 * cb + c16;
+                row[cb] = (size_t)(n < N ? n : N - 1) + (half ? (size_t)N : 0);
+            }
 #pragma unroll 1
-                for (int w = 0; w < K / 8; w++) {
-                    const uint32_t g = (uint32_t)(w * 8) >> gshift, word = qw[row * (K / 8) + w];
-                    const int z = qz ? (int)((qz[row * ZW + (g >> 3)] >> (4 * (g & 7))) & 15u) : 8;
-                    const float scale = f16_dev(scales[row * G + g]);
-#pragma unroll 1
-                    for (int t = 0; t < 8; t++)
-                        f += bf16_to_f32(x[mc * K + w * 8 + t]) * ((float)((int)((word >> (4 * t)) & 15u) - z) * scale);
+            for (int i = 0; i < MT; i++) {
+                const uint16_t* xr[RB];
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++) {
+                    const int m = m0 + i * MR + 16 * rb + c16;
+                    xr[rb] = x + (size_t)(m < M ? m : M - 1) * (size_t)K + 8 * q16;
                 }
+                f32x4 sum[RB][2] = {};
+#pragma unroll 1
+                for (int u = 0; u < K / GS; u++) {
+                    const uint32_t g = (uint32_t)(u * GS) >> gshift;
+                    f32x4 acc[RB][2] = {};
+                    int z[2];
+                    float sc[2];
 #pragma unroll
-                for (int o = 0; o < OWN; o++)
+                    for (int cb = 0; cb < 2; cb++) {
+                        z[cb] = qz ? (int)((qz[row[cb] * ZW + (g >> 3)] >> (4 * (g & 7))) & 15u) : 8;
+                        sc[cb] = f16_dev(scales[row[cb] * G + g]) * 65536.0f;
+                    }
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        if (it == o * 4 + e && !finite(res[o][e])) res[o][e] = f;
-                        if (it == (OWN + o) * 4 + e && !finite(up[o][e])) up[o][e] = f;
+                    for (int j = 0; j < GS / 32; j++) {
+                        bf16x8 a[RB];
+#pragma unroll
+                        for (int rb = 0; rb < RB; rb++) a[rb] = *reinterpret_cast<const bf16x8*>(xr[rb] + u * GS + 32 * j);
+#pragma unroll
+                        for (int cb = 0; cb < 2; cb++) {
+                            const uint32_t word = qw[row[cb] * (size_t)(K / 8) + (u * GS / 8 + 4 * j + q16)];
+                            u32x4 c;
+#pragma unroll
+                            for (int t = 0; t < 4; t++) {
+                                const float lo = (float)((int)((word >> (8 * t)) & 15u) - z[cb]) * 0x1p-16f;
+                                const float hi = (float)((int)((word >> (8 * t + 4)) & 15u) - z[cb]) * 0x1p-16f;
+                                c[t] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
+                            }
+#pragma unroll
+                            for (int rb = 0; rb < RB; rb++) acc[rb][cb] = mfma_of<16>::mul(a[rb], __builtin_bit_cast(bf16x8, c), acc[rb][cb]);
+                        }
+                    }
+#pragma unroll
+                    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+                        for (int cb = 0; cb < 2; cb++)
+#pragma unroll
+                            for (int e = 0; e < 4; e++) sum[rb][cb][e] = __builtin_fmaf(sc[cb], acc[rb][cb][e], sum[rb][cb][e]);
+                }
+                // rows 4 q16 .. + 3 of column c16 of a block, to the places in LDS of the
+                // wave's own pieces (which no other wave reads) in the order of res
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+                    for (int cb = 0; cb < 2; cb++) {
+                        const int piece = MR == 32 ? MT * (2 * rb + (q16 >> 1)) + i : cb;
+                        const int to = MR == 32 ? 32 * (q16 & 1) + 16 * cb + c16 : lane;
+                        if (piece % KW == kw) red[piece * 64 + to - lane] = sum[rb][cb];
                     }
             }
-        }
-    }
-
-    // rows past M lie past the buffer's records and are dropped there; lanes
-    // of columns past N take an offset that is
-    const uint32_t eb = y_f32 ? 4 : 2;
-    const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(y, (short)0, (int)((uint32_t)M * (uint32_t)N * eb), 0x00020000);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-    for (int o = 0; o < OWN; o++) {
-        const int p = kw + o * KW;
-        const int s = p % NS, i = (p / NS) % MT, v = p / (NS * MT);
-        const int n = c0 + s * MR + r, m = m0 + i * MR + (MR == 32 ? 8 * v + 4 * q : 4 * q);
-        uint32_t off = n < N ? ((uint32_t)m * (uint32_t)N + (uint32_t)n) * eb : 0x80000000u;
-        if (bias) res[o] += bias[n < N ? n : N - 1];
-        if (glu) {
-            if (bias) up[o] += bias[N + (n < N ? n : N - 1)];
+            for (int o = 0; o < OWN; o++) {
+                const f32x4 f = red[(kw + o * KW) * 64];
+                float a[4], b[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) res[o][e] = silu_mul_fast(res[o][e], up[o][e]);
-        }
-        if (y_f32) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float f = res[o][e];
-                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, f), ry, off, 0, 0);
-                off += (uint32_t)N * 4u;
+                for (int e = 0; e < 4; e++) {
+                    a[e] = half || __builtin_isfinite(res[o][e]) ? res[o][e] : f[e];
+                    b[e] = !half || __builtin_isfinite(up[o][e]) ? up[o][e] : f[e];
+                }
+                res[o] = f32x4{a[0], a[1], a[2], a[3]};
+                up[o] = f32x4{b[0], b[1], b[2], b[3]};
             }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                __builtin_amdgcn_raw_buffer_store_b16(bf16_out(res[o][e]), ry, off, 0, 0);
-                off += (uint32_t)N * 2u;
-            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
+        finish();
+        return;
     }
+    finish();
 }
 
 struct Batch {
