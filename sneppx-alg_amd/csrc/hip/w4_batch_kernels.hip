@@ -493,7 +493,7 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
         }
     };
 
-    // Groups below 128: an infinite activation (or one past 1e37) makes both products infinite and
+    // An infinite activation (or one past 1e37) makes both products infinite and
     // their difference NaN where sum x (q - z) s is an infinity or a number.  A
     // wave with a result that is not finite computes its columns once more in
     // that form, straight from memory, and takes from it what was not finite:
@@ -501,9 +501,9 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
     // 32 rows at a time, as K / GS round trips to memory whatever the number of
     // such results.  N = 6144, K = 4096, groups of 64, M = 96: 0.29 ms with one
     // row of them, 0.51 with 96 (k_w4a16_generic, which these groups ran before,
-    // 2.7).  It stores its results itself: calls without such results then pay for
-    // the test alone (18.5 us at 96 rows; 18.9 where the two ways met before the
-    // stores).
+    // 2.7); N = 4096, K = 11008, groups of 128: 0.59 and 0.97 (7.6).  It stores
+    // its results itself: calls without such results then pay for the test alone
+    // (0.1 us at 96 rows; 0.8 where the two ways met before the stores).
     f32x4 odd = {};                 // NaN where a result is not finite
 #pragma unroll
     for (int o = 0; o < OWN; o++)
@@ -516,7 +516,7 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
             for (int e = 0; e < 4; e++) odd[e] = __builtin_fmaf(0.0f, up[o][e], odd[e]);
     }
     const float any = (odd[0] + odd[1]) + (odd[2] + odd[3]);
-    if (GS < 128 && __builtin_expect(__ballot(any != any) != 0, 0)) {
+    if (__builtin_expect(__ballot(any != any) != 0, 0)) {
         constexpr int RB = MR / 16;             // blocks of 16 rows, by two of 16 columns
         const int c16 = lane & 15, q16 = lane >> 4;
 #pragma unroll 1

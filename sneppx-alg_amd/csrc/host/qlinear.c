@@ -169,13 +169,16 @@ static size_t w4_prep_bytes(size_t M, size_t K) {
  * split K): where it may and the batch kernel is not estimated to be faster by a
  * tenth (what the estimates are off by).
  * Below SNX_W4_GEMM_MIN_M only where the allocation-free entry point, which
- * decides alike, has the scratch for it.  recorded: the call is captured into
+ * decides alike, has the scratch for it, and with K in whole 512s: the GEMM
+ * gives NaN where an infinite activation makes the result infinite, as the
+ * decode GEMV of those shapes does, and the batch kernel does not.  recorded: the call is captured into
  * a graph and neither the batch kernel nor a smaller GEMM is a choice. */
 static int w4_takes_gemm(size_t M, size_t N, size_t K, int group, const uint16_t* scales, const uint32_t* qzeros,
                          int y_f32, int glu, int recorded) {
     if (M < (y_f32 || recorded ? SNX_W4_GEMM_MIN_M : SNX_W4_GEMM_MIN_M_BF16) || ((uintptr_t)scales & 3u) != 0 ||
         ((uintptr_t)qzeros & 3u) != 0 || !snx_w4a16_gemm_ok(M, N, K, group) ||
-        (M < SNX_W4_GEMM_MIN_M && w4_prep_bytes(M, K) > SNEPPX_NOALLOC_SCRATCH_BYTES))
+        (M < SNX_W4_GEMM_MIN_M &&
+         (w4_prep_bytes(M, K) > SNEPPX_NOALLOC_SCRATCH_BYTES || !snx_w4a16_gemv_supported(64, N, K, group))))
         return 0;
     return recorded || !snx_w4a16_batch_ok(M, N, K, group, scales, qzeros) ||
            10 * snx_w4a16_gemm_cost(M, N, K, glu ? 1 : snx_w4a16_gemm_splits(M, N, K)) <= 11 * snx_w4a16_batch_cost(M, N, K);
