@@ -124,14 +124,14 @@ int SNEPPX_qlinear_w4a16(const uint16_t* x, const uint32_t* qweight, const uint1
  * reference).  For callers that cannot allocate device memory: code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.
  * Same arguments, dispatch and results (bit-identical) as
- * SNEPPX_qlinear_w4a16, with one exception: where the allocating entry point
+ * SNEPPX_qlinear_w4a16, with two exceptions.  Where the allocating entry point
  * splits the prefill GEMM's K into spans (few output tiles, e.g. one GPU's
  * tensor-parallel QKV shard, or the tiles past the last full round of CUs,
  * e.g. the Llama-3-8B QKV projection at 1849 tokens), this one runs that
- * GEMM whole-K, the same
+ * GEMM whole-K, or the batch kernel where that is the faster one: the same
  * product with another fp32 summation order, so a bf16 output can differ
- * in its last bit; and a call recorded into a graph takes the batch kernel
- * here, and kernels without scratch there.  The scratch the split-K decode and the prefill
+ * in its last bit.  And a call recorded into a graph can take the batch kernel
+ * here, and does not there.  The scratch the split-K decode and the prefill
  * GEMM need (fp32 partials, prepared activations) comes from one static
  * device array of SNEPPX_NOALLOC_SCRATCH_BYTES per GPU, held from the first
  * call on that GPU until the process ends, instead of a workspace.  A call

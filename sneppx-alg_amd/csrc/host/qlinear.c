@@ -165,23 +165,26 @@ static size_t w4_prep_bytes(size_t M, size_t K) {
     return ((M * K * sizeof(uint16_t) + 255) & ~(size_t)255) + (K / 128) * snx_w4_prep_rows(M) * sizeof(float);
 }
 
-/* Whether M x N x K runs the prefill GEMM (glu: its SwiGLU form, which does not
- * split K): where it may and the batch kernel is not estimated to be faster by a
- * tenth (what the estimates are off by).
- * Below SNX_W4_GEMM_MIN_M only where the allocation-free entry point, which
- * decides alike, has the scratch for it, and with K in whole 512s: the GEMM
- * gives NaN where an infinite activation makes the result infinite, as the
- * decode GEMV of those shapes does, and the batch kernel does not.  recorded: the call is captured into
- * a graph and neither the batch kernel nor a smaller GEMM is a choice. */
+/* Whether M x N x K runs the prefill GEMM (whole_k: not in spans of K, as its
+ * SwiGLU form and the allocation-free entry point run it): where it may and the
+ * batch kernel is not estimated to be faster by a tenth (what the estimates are
+ * off by).  N = 4096, K = 14336, M = 193: 66 us in spans, 173 whole-K, the batch
+ * kernel 66.
+ * Below SNX_W4_GEMM_MIN_M only where the allocation-free entry point has the
+ * scratch for it, and with K in whole 512s: the GEMM gives NaN where an infinite
+ * activation makes the result infinite, as the decode GEMV of those shapes does,
+ * and the batch kernel does not.
+ * recorded: the call is captured into a graph and neither the batch kernel nor a
+ * smaller GEMM is a choice. */
 static int w4_takes_gemm(size_t M, size_t N, size_t K, int group, const uint16_t* scales, const uint32_t* qzeros,
-                         int y_f32, int glu, int recorded) {
+                         int y_f32, int whole_k, int recorded) {
     if (M < (y_f32 || recorded ? SNX_W4_GEMM_MIN_M : SNX_W4_GEMM_MIN_M_BF16) || ((uintptr_t)scales & 3u) != 0 ||
         ((uintptr_t)qzeros & 3u) != 0 || !snx_w4a16_gemm_ok(M, N, K, group) ||
         (M < SNX_W4_GEMM_MIN_M &&
          (w4_prep_bytes(M, K) > SNEPPX_NOALLOC_SCRATCH_BYTES || !snx_w4a16_gemv_supported(64, N, K, group))))
         return 0;
     return recorded || !snx_w4a16_batch_ok(M, N, K, group, scales, qzeros) ||
-           10 * snx_w4a16_gemm_cost(M, N, K, glu ? 1 : snx_w4a16_gemm_splits(M, N, K)) <= 11 * snx_w4a16_batch_cost(M, N, K);
+           10 * snx_w4a16_gemm_cost(M, N, K, whole_k ? 1 : snx_w4a16_gemm_splits(M, N, K)) <= 11 * snx_w4a16_batch_cost(M, N, K);
 }
 
 /* One row, and M <= 4 within the LDS-staged small-M kernel (groups of 256 and
@@ -242,7 +245,7 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
     if (noalloc && aligned && !snx_noalloc_scratch(w4_noalloc_bytes(M, N, K, group, scales, qzeros), who)) return -1;
     /* (a call of the M = 1 kernels takes no workspace, and is not asked about) */
     const int recorded = !noalloc && !(M == 1 && w4_small(M, K, group, scales, qzeros)) && snx_stream_capturing(stream);
-    if (aligned && w4_takes_gemm(M, N, K, group, scales, qzeros, y_f32, 0, recorded)) {
+    if (aligned && w4_takes_gemm(M, N, K, group, scales, qzeros, y_f32, noalloc, recorded)) {
         /* prefill GEMM: activations prepared once into the call's scratch */
         const size_t Mp = snx_w4_prep_rows(M);
         const size_t xp_bytes = (M * K * sizeof(uint16_t) + 255) & ~(size_t)255;
