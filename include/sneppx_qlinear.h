@@ -138,15 +138,21 @@ int SNEPPX_qlinear_w4a16(const uint16_t* x, const uint32_t* qweight, const uint1
  * that needs more scratch than that returns -1 with the reason (for
  * example split-K partials K/1024 * M * N * 4 bytes, prefill 2 M K bytes and
  * more).  Every call on a GPU shares its array: calls that overlap on one GPU
- * (two streams, two threads) race on it and must be serialised by the
- * caller; beside it lie arrival counters that every call leaves at zero, which
- * an overlap can leave otherwise.  Nothing in the array needs to start at zero. */
+ * (two streams, two threads, replays of a graph) race on it and must be
+ * serialised by the caller.  Nothing in the array needs to start at zero, but
+ * beside it lie arrival counters that every call finds and leaves at zero: an
+ * overlap can leave one otherwise, and then later calls that use it give wrong
+ * results too, also one by one, until SNEPPX_qlinear_noalloc_reset. */
 #define SNEPPX_NOALLOC_SCRATCH_BYTES (32u << 20)
 int SNEPPX_qlinear_w4a16_noalloc(const uint16_t* x, const uint32_t* qweight,
                                  const uint16_t* scales, const uint32_t* qzeros,
                                  const int32_t* g_idx, size_t G, const float* bias, void* y,
                                  SNEPPXDtype y_dtype, size_t M, size_t N, size_t K, int group,
                                  SNEPPXStream stream);
+/* Zeroes the current GPU's arrival counters of the call above, ordered on
+ * `stream`, with no such call running: for a caller that has let calls overlap.
+ * Returns 0, or -1 with the reason. */
+int SNEPPX_qlinear_noalloc_reset(SNEPPXStream stream);
 
 /* C3 fast path, step 1 (once per layer, at load time): GPTQ act-order
  * weights (qweight in column order k, g_idx int32 [K]) -> group-contiguous

@@ -43,14 +43,9 @@ namespace {
 void* ws_alloc(size_t bytes, void* stream, bool zeroed) {
     void* p = nullptr;
     if (snx_hip_malloc_async(&p, bytes, stream)) return nullptr;
-    if (zeroed) {
-        const size_t n = bytes / 4;
-        k_fill_zero_u32<<<(unsigned)(n / 256 < 1024 ? (n + 255) / 256 : 1024), 256, 0, S(stream)>>>(
-            static_cast<uint32_t*>(p), n);
-        if (snx_launch_check("k_fill_zero_u32")) {
-            (void)hipFreeAsync(p, S(stream));
-            return nullptr;
-        }
+    if (zeroed && snx_k_fill_zero(p, bytes, stream)) {
+        (void)hipFreeAsync(p, S(stream));
+        return nullptr;
     }
     return p;
 }
@@ -111,6 +106,13 @@ const char* SNEPPX_qlinear_last_error(void) { return g_err; }
 
 int snx_launch_check(const char* kernel) {
     return check(hipGetLastError(), kernel);
+}
+
+int snx_k_fill_zero(void* p, size_t bytes, void* stream) {
+    const size_t n = bytes / 4;
+    k_fill_zero_u32<<<(unsigned)(n / 256 < 1024 ? (n + 255) / 256 : 1024), 256, 0, S(stream)>>>(
+        static_cast<uint32_t*>(p), n);
+    return snx_launch_check("k_fill_zero_u32");
 }
 
 int snx_hip_device_count(int* count) {

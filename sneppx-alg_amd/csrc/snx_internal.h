@@ -38,6 +38,8 @@ void* snx_noalloc_scratch(size_t bytes, const char* who);
 void* snx_noalloc_counters(size_t bytes, const char* who);
 void snx_clear_error(void);
 int snx_launch_check(const char* kernel);
+/* zeroes bytes / 4 words (a kernel, not a memset) */
+int snx_k_fill_zero(void* p, size_t bytes, void* stream);
 
 /* kinds of snx_k_finalize_scale */
 enum {

@@ -151,6 +151,7 @@ EXPORTS = {
     "snx_hip_stream_sync": (C.c_int, [_vp]),
     "snx_hip_device_info": (C.c_int, [C.c_char_p, _sz, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "SNEPPX_qlinear_release_workspaces": (C.c_int, [_vp]),
+    "SNEPPX_qlinear_noalloc_reset": (C.c_int, [_vp]),
     "SNEPPX_qlinear_w8a8_i8_dyn": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _vp]),
     "SNEPPX_qlinear_w8a8_fp8_dyn": (C.c_int, [_vp, _vp, _vp, _vp, _vp, _sz, _sz, _sz, _vp]),
     "snx_hip_stream_begin_capture": (C.c_int, [_vp]),
@@ -389,6 +390,11 @@ class Library:
         self.check(self.fn["SNEPPX_qlinear_w4a16_noalloc"](
             _ptr(x), _ptr(qweight), _ptr(scales), _ptr(qzeros), _ptr(g_idx), G, _bias_ptr(bias, N, y), _ptr(y),
             ydt, M, N, K, group, self._stream(stream)), "qlinear_w4a16_noalloc")
+
+    def qlinear_noalloc_reset(self, stream=None):
+        """SNEPPX_qlinear_noalloc_reset: for a program that has let calls of
+        qlinear_w4a16_noalloc overlap."""
+        self.check(self.fn["SNEPPX_qlinear_noalloc_reset"](self._stream(stream)), "qlinear_noalloc_reset")
 
     def qlinear_w4_actorder_prepare(self, qweight, g_idx, G, qweight_sorted, perm, stream=None):
         N, K8 = qweight.shape
