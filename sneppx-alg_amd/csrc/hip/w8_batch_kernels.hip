@@ -3,14 +3,18 @@
 //
 // y[m][n] = s[n] * sum_k x[m][k] * q[n][k] (+ bias[n]), q int8.
 //
-// An fp32 value is exactly the sum of three bf16 values (its 24 significant
-// bits cut into 8 + 8 + 8) and an int8 is exactly one, so three bf16 products
-// with fp32 accumulation compute what fp32 arithmetic does.  1. k_w8_split_x
-// writes the pieces once; 2. k_w8_batch multiplies.  The leading pieces'
-// products meet in accumulators that are added to the result every 128
-// columns, the others' (a 256th of the size) in their own: the sum's error
-// stays that of short fp32 chains, 9e-8 at K = 4096 (the fp32 kernel's is
-// 1.6e-7).  Measured at N = K = 4096 (before: k_w8_gemv, one row after the
+// An fp32 value is exactly p0 + 2^-8 p1 + 2^-16 p2 with bf16 p0, p1, p2 (its 24
+// significant bits cut into 8 + 8 + 8, the later pieces scaled up so that they
+// are bf16 values also where x is tiny or subnormal) and an int8 is exactly
+// one, so three bf16 products with fp32 accumulation compute what fp32
+// arithmetic does.  1. k_w8_split_x writes the pieces once; 2. k_w8_batch
+// multiplies.  The leading pieces' products meet in accumulators that are added
+// to the result every 128 columns, the second and third ones' (with their
+// scales a 256th and a 65536th of the size) in their own: the sum's error stays
+// that of short fp32 chains, 7e-8 at K = 2048 for activations of any size down to
+// 1e-40 (the fp32 kernel's is 1.3e-7).  Pieces that are not scaled share one
+// accumulator (53.5 against 53.8 us at 384 rows), but lose the low bits of x
+// below 2^-110 and all of it below 2^-133.  Measured at N = K = 4096 (before: k_w8_gemv, one row after the
 // other on the vector units): M = 16 94 -> 15.6 us, 64 371 -> 19.3, 384
 // 2490 -> 58.
 #include <hip/hip_runtime.h>
@@ -48,9 +52,9 @@ __device__ __forceinline__ void lds_load16(__amdgpu_buffer_rsrc_t r, void* dst, 
 
 // ------------------------------------------------------- activation pieces
 // xp [M][steps][3][64] bf16: piece p of the 64 columns of a step, zero past K.
-// One thread per 4 columns; each piece is the top 16 bits of what is left
-// (cut, not rounded: no piece overflows, and the third is exact).  An infinity
-// or NaN is its first piece alone.
+// One thread per 4 columns; each piece is the top 16 bits of what is left, times
+// 2^8 after each (cut, not rounded: no piece overflows, and the third is exact).
+// An infinity or NaN is its first piece alone.
 __global__ void __launch_bounds__(256) k_w8_split_x(const float* __restrict__ x, uint16_t* __restrict__ xp, int K,
                                                     uint32_t items, uint32_t per_row) {
     const uint32_t it = blockIdx.x * 256 + threadIdx.x;
@@ -70,7 +74,7 @@ __global__ void __launch_bounds__(256) k_w8_split_x(const float* __restrict__ x,
         for (int i = 0; i < 3; i++) {
             const uint32_t hi = f2u(v) & 0xFFFF0000u;
             p[i][e >> 1] |= (e & 1) ? hi : hi >> 16;
-            v -= u2f(hi);       // exact: the bits that were cut off
+            v = (v - u2f(hi)) * 256.0f;     // exact: the bits that were cut off
         }
     }
     uint16_t* o = xp + ((size_t)m * (per_row / 16) + k / BK) * (3 * BK) + k % BK;
@@ -155,9 +159,10 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
             lds_load16(rq, st + L::A + nw * 2048 + i * 1024, gb[i], (g0 + t) * BK);
     };
 
-    f32x16 yv[MT], al[MT], ah[MT];      // the result, the small pieces' sums, the leading ones' of 128 columns
+    // the result, the leading pieces' sums of 128 columns, the second and third ones'
+    f32x16 yv[MT], ah[MT], am[MT], al[MT];
 #pragma unroll
-    for (int i = 0; i < MT; i++) yv[i] = al[i] = ah[i] = f32x16{};
+    for (int i = 0; i < MT; i++) yv[i] = ah[i] = am[i] = al[i] = f32x16{};
 
     // what a step reads from its stage ahead of its products
     u32x4 wd[2];
@@ -207,7 +212,7 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
 #pragma unroll
             for (int i = 0; i < MT; i++) {
                 ah[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0][i], fb, ah[i], 0, 0, 0);
-                al[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[1][i], fb, al[i], 0, 0, 0);
+                am[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[1][i], fb, am[i], 0, 0, 0);
                 al[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[2][i], fb, al[i], 0, 0, 0);
             }
         };
@@ -249,7 +254,10 @@ __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(K
         }
     }
 #pragma unroll
-    for (int i = 0; i < MT; i++) yv[i] += al[i];
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+            yv[i][e] = __builtin_fmaf(__builtin_fmaf(al[i][e], 0x1p-8f, am[i][e]), 0x1p-8f, yv[i][e]);
 
     // piece p = MT v + i: rows 8 v + 4 h .. + 3 of tile i.  The wave groups'
     // sums meet in LDS and wave (nw, kw) finishes pieces kw, kw + KW, ...

@@ -4,7 +4,7 @@ of the 128-column tiles, widths that are no multiple of a 64-column step or of
 16 bytes, one span of K and many, bias, and activations of unlike magnitude,
 signed zero, infinities and NaN.
 
-The pieces hold every bit of an fp32 activation and an int8 is one bf16, so
+The pieces hold every bit of an fp32 activation, subnormal ones too, and an int8 is one bf16, so
 only the fp32 accumulation rounds: chains of 128 columns and of K / 128 partial
 sums, each rounding 2^-24 of a value a few times the result's size.  2e-6 of
 the largest result is over ten times the expected random walk."""
@@ -53,9 +53,11 @@ def test_w8_batch_every_bit_of_an_activation_counts(lib):
     print("[gpu] w8 batch single activations", flush=True)
     K, M = 256, 64
     rng = np.random.default_rng(3)
-    vals = rng.integers(1 << 20, 0x7F000000, M).astype(np.uint32).view(np.float32)   # every magnitude from 2^-118 up
+    bits = rng.integers(1, 0x7F800000, M).astype(np.uint32)     # magnitudes of every size
+    bits[4:24] = rng.integers(1, 1 << 25, 20)                   # subnormal and nearly so
+    bits[24:48] = rng.integers(1 << 25, 1 << 28, 24)            # up to 2^-95
+    vals = bits.view(np.float32)
     vals[:4] = [1.0 + 2.0**-23, -(2.0 - 2.0**-23), 3.4028234663852886e38, -0.0]
-    vals = np.where(np.abs(vals) < 2.0**-100, np.float32(1.5), vals)
     x = np.zeros((M, K), np.float32)
     x[np.arange(M), rng.integers(0, K, M)] = vals
     q = np.where(np.arange(2)[:, None] == 0, 1, -1).astype(np.int8) * np.ones((2, K), np.int8)
@@ -78,3 +80,16 @@ def test_w8_batch_non_finite_activations(lib):
     assert np.array_equal(np.sign(y[np.isinf(y)]), np.sign(want[np.isinf(want)]))
     fine = np.isfinite(want)
     assert rel_err(y[fine], want[fine]) <= 2e-6
+
+
+@pytest.mark.parametrize("size", [1e-30, 1e-34, 1e-36, 1e-38, 1e-40])
+def test_w8_batch_tiny_activations(lib, size):
+    """Rows of a size where bf16 has few bits or none: the error of any other rows,
+    and half a unit of the smallest fp32 for results that small."""
+    print(f"[gpu] w8 batch activations of {size}", flush=True)
+    rng = np.random.default_rng(11)
+    x = (rng.normal(0, 1, (48, 2048)) * size).astype(np.float32)
+    q = rng.integers(-128, 128, (300, 2048)).astype(np.int8)
+    want = x.astype(np.float64) @ q.astype(np.float64).T
+    y = _run(lib, x, q, np.ones(300, np.float32))
+    assert np.abs(y - want).max() <= 2e-6 * np.abs(want).max() + 2.0**-149
