@@ -197,15 +197,33 @@ static int w4_small(size_t M, size_t K, int group, const uint16_t* scales, const
 }
 
 /* Shapes with little to stream, where the start and the meeting of the batch
- * kernel's spans weigh most.  17 to 32 rows with K up to 1024: the decode GEMV,
- * 4.3 against 5.0 us at N = 4096, K = 512, M = 32 and 6.1 against 7.6 at K =
- * 1024 (N = 14336, K = 512: 7.8 against 5.8).  2 to 16 rows with K from 8192 in
- * few split-K spans and N up to 1536: split-K, 11.2 against 12.7 us at N = 1408,
- * K = 8192, M = 8 and 12.3 against 13.4 at N = 961, K = 13312 (N = 2048: 15.0
- * against 14.1; in spans of 256, K = 11008: 23.4 against 12.8). */
-static int w4_short(size_t M, size_t N, size_t K, int group) {
-    return M > 16 ? M <= 32 && K <= 1024 && N <= 4096 && snx_w4a16_gemv_supported(M, N, K, group)
-                  : M > 1 && K >= 8192 && N <= 1536 && snx_w4a16_splitk_span(M, K, group) >= 512;
+ * kernel's spans weigh most (us of the other kernel / the batch kernel).
+ * 17 rows and more, the decode GEMV, while its workgroups of 16 columns are few:
+ *   M = 17, 32, K = 512: N = 4096 - , 4.3 / 5.0; 6144 4.2 / 4.8, 4.8 / 4.9;
+ *                        8192 4.3 / 4.8, 4.9 / 5.0; 10240 5.1 / 4.9, 6.0 / 4.9
+ *   K = 1024:            N = 4096 - , 6.1 / 7.6; 6144 5.8 / 7.2, 7.0 / 7.4;
+ *                        8192 5.9 / 7.3, 7.0 / 7.4; 10240 7.0 / 7.6, 9.1 / 7.5
+ *   K = 1536:            N = 4096 6.6 / 7.7, 7.5 / 7.7; 8192 7.6 / 8.1, 9.3 / 8.3
+ *   K = 2048, N = 4096:  M = 17 7.9 / 8.5, 28 8.2 / 8.5, 32 8.6 / 8.5
+ *   M = 33, 48, 64, K = 512: N = 4096 5.3 / 6.2, 5.7 / 6.3, 6.3 / 6.3 (fp32 5.9 / 6.4);
+ *                        8192 5.8 / 6.3, 6.3 / 6.3, 7.5 / 6.3
+ *   K = 1024:            N = 4096 7.4 / 8.3, 7.8 / 8.3, 9.0 / 8.4; 6144 8.6 / 8.6
+ * 2 to 16 rows, split-K in few spans: K = 7168, N = 512 9.8 / 9.5, 1024 10.0 / 10.6,
+ * 2048 10.0 / 10.9, 2560 11.9 / 11.5; K = 8192, N = 1408 11.2 / 12.7, 2048 10.7 / 12.2,
+ * 2560 13.4 / 12.5; K = 9216, N = 2048 12.4 / 12.4; N = 961, K = 13312 12.3 / 13.4 (in
+ * spans of 256, K = 11008: 23.4 / 12.8).
+ * glu: stacked gate/up rows, where the other kernel needs the rule's own pass:
+ * K = 512, N = 4096 6.0 / 5.0, but K = 1024 7.0 / 7.5, K = 10240, N = 1536 12.7 / 13.9. */
+static int w4_short(size_t M, size_t N, size_t K, int group, int glu) {
+    if (M > 16) {
+        if (!snx_w4a16_gemv_supported(M < 64 ? M : 64, N, K, group)) return 0;
+        if (glu) return M <= 32 && K <= 1024 && N <= 4096;
+        if (M <= 19 && N <= (K <= 1024 ? 10240u : K <= 1536 ? 8192u : 4096u) && K <= 2048) return 1;
+        if (M <= 32) return N <= 8192 && (K <= 1024 || (N <= 4096 && (K <= 1536 || (K <= 2048 && M <= 28))));
+        return (M <= 48 && K <= 1024 && N <= 4096) || (M <= 64 && K <= 512 && N <= (M <= 48 ? 8192u : 4096u));
+    }
+    if (M < 2 || snx_w4a16_splitk_span(M, K, group) < 512) return 0;
+    return (K >= 8192 && N <= 1536) || (!glu && K >= 7168 && K <= 8192 && N >= 1024 && N <= 2048);
 }
 
 /* The scratch that SNEPPX_qlinear_w4a16_noalloc is documented to need:
@@ -271,7 +289,7 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
         /* 2 <= M <= 16: one persistent workgroup per CU, activations staged once */
         return snx_k_w4a16_gemv_mt(x, qweight, scales, qzeros, NULL, y, bias, y_f32, M, N, K, stream);
     }
-    if (aligned && !recorded && !w4_small(M, K, group, scales, qzeros) && !w4_short(M, N, K, group) &&
+    if (aligned && !recorded && !w4_small(M, K, group, scales, qzeros) && !w4_short(M, N, K, group, 0) &&
         snx_w4a16_batch_ok(M, N, K, group, scales, qzeros))
         return w4_batch(who, noalloc, x, qweight, scales, qzeros, bias, y, y_f32, M, N, K, group, 0, stream);
     const int kspan = snx_w4a16_splitk_span(M, K, group);
@@ -425,7 +443,7 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
     /* (up to 8 rows of the persistent decode kernel's shapes its fp32 rows and
      * the rule's own pass stay faster: 20.8 against 22.5 us at F = 14336) */
     if (aligned && !recorded && !(M <= 8 && snx_w4a16_mt_ok(M, K, group, 0)) && !(M == 1 && w4_small(M, K, group, scales, qzeros)) &&
-        !w4_short(M, 2 * F, K, group) &&
+        !w4_short(M, 2 * F, K, group, 1) &&
         snx_w4a16_batch_ok(M, 2 * F, K, group, scales, qzeros))
         return w4_batch("qlinear_w4a16_swiglu", 0, x, qweight, scales, qzeros, bias, out, 0, M, F, K, group, 1, stream);
     /* other shapes: the [M][2F] projection in fp32 scratch, then the same rule */

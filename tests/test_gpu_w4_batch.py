@@ -41,9 +41,9 @@ def _case(oracle, N, K, group, zeros, seed):
     (5, 38, 4224, 128, False, True, "f32"),       # 33 steps in spans of unlike length, column tail
     (5, 37, 4224, 128, True, False, "f32"),       # an odd number of scales
     (40, 1, 384, 128, False, False, "f32"),       # three scales
-    (16, 300, 8192, 256, True, False, "bf16"),    # a full 16-row block, many spans
+    (16, 300, 6144, 256, True, False, "bf16"),    # a full 16-row block, many spans
     (16, 65, 1152, 32, True, False, "f32"),
-    (17, 129, 1024, 128, True, True, "f32"),      # one past a 16-row block
+    (17, 129, 1152, 128, True, True, "f32"),      # one past a 16-row block
     (32, 256, 640, 64, False, False, "f32"),
     (33, 96, 2048, 128, True, False, "f32"),      # 64-row block with a tail
     (64, 1000, 512, 32, True, True, "bf16"),
