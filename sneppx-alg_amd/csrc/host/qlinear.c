@@ -423,6 +423,9 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
     REQUIRE(aligned16(out), "qlinear_w4a16_swiglu: out must be 16-byte aligned");
     snx_clear_error();
     const int aligned = aligned16(x) && aligned16(qweight);
+    /* one decode row: gate and up rows of an output in one wave, SwiGLU on its total */
+    if (M == 1 && aligned && snx_w4a16_gemv1_swiglu_ok(F, K, group, scales, qzeros))
+        return snx_k_w4a16_gemv1_swiglu(x, qweight, scales, qzeros, bias, out, F, K, group, stream);
     const int recorded = snx_stream_capturing(stream);
     if (aligned && w4_takes_gemm(M, 2 * F, K, group, scales, qzeros, 0, 1, recorded)) {
         const size_t Mp = snx_w4_prep_rows(M);
@@ -436,10 +439,6 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
                                               group, Mp, stream);
         return rc;
     }
-    /* one decode row: gate and up rows of an output in one wave, SwiGLU on its total */
-    if (M == 1 && aligned16(x) && aligned16(qweight) &&
-        snx_w4a16_gemv1_swiglu_ok(F, K, group, scales, qzeros))
-        return snx_k_w4a16_gemv1_swiglu(x, qweight, scales, qzeros, bias, out, F, K, group, stream);
     /* (up to 8 rows of the persistent decode kernel's shapes its fp32 rows and
      * the rule's own pass stay faster: 20.8 against 22.5 us at F = 14336) */
     if (aligned && !recorded && !(M <= 8 && snx_w4a16_mt_ok(M, K, group, 0)) && !(M == 1 && w4_small(M, K, group, scales, qzeros)) &&
@@ -471,7 +470,7 @@ int SNEPPX_qlinear_w4a16_mlp(const uint16_t* x, const uint32_t* gu_qweight, cons
     REQUIRE(y_dtype == SNEPPX_BFLOAT16 || y_dtype == SNEPPX_FLOAT32,
             "qlinear_w4a16_mlp: y_dtype must be SNEPPX_BFLOAT16 or SNEPPX_FLOAT32");
     snx_clear_error();
-    const int recorded = snx_stream_capturing(stream);
+    const int recorded = M >= SNX_W4_GEMM_MIN_M_BF16 && snx_stream_capturing(stream);
     if (aligned16(x) && aligned16(gu_qweight) && aligned16(dn_qweight) && F % 128 == 0 &&
         w4_takes_gemm(M, 2 * F, H, group, gu_scales, gu_qzeros, 0, 1, recorded) &&
         w4_takes_gemm(M, N, F, group, dn_scales, dn_qzeros, y_dtype == SNEPPX_FLOAT32, 0, recorded)) {
