@@ -428,9 +428,19 @@ int snx_q8_batch_ok(int kind, size_t M, size_t N, size_t K) {
 // Where the 256 x 224 tiles of gemm_kernels.hip apply too (M, N >= 128), the
 // batch kernel is the faster one while its own largest tiles are one round of
 // the CUs: int8 at N = 14336, K = 4096 31 against 43 us at M = 256, equal at
-// 512 (mxfp8 36 / 62 and 64 / 63); at N = K = 4096 30 / 42 at M = 1024.
+// 512 (mxfp8 36 / 62 and 64 / 63); at N = K = 4096 30 / 42 at M = 1024.  The MX
+// formats of 8 and 6 bits have those tiles for fewer rows too, and take them where
+// they are half the rounds of the CUs (mxfp8, K = 4096, M = 100: N = 36864 67 / 59 us,
+// 49152 69 / 63, 57344 71 / 66, 65536, where both are two rounds, 76 / 118; M = 32:
+// 36864 54 / 53).
 int snx_q8_batch_better(int kind, size_t M, size_t N, size_t K) {
-    return snx_q8_batch_ok(kind, M, N, K) && (M < 128 || N < 128 || tiles_of(M, N, 128) <= (size_t)snx::cu_count());
+    const size_t ncu = (size_t)snx::cu_count();
+    if (!snx_q8_batch_ok(kind, M, N, K)) return 0;
+    if (M >= 128 && N >= 128) return tiles_of(M, N, 128) <= ncu;
+    if (kind < MX || kind == 6 || M <= 32) return 1;
+    const size_t rounds = (tiles_of(M, N, rows_of(kind, M, N)) + ncu - 1) / ncu;
+    const size_t large = ((M + 255) / 256 * ((N + 223) / 224) + ncu - 1) / ncu;
+    return rounds < 2 * large;
 }
 
 int snx_k_q8_batch(int kind, const void* A, const void* sA, const void* W, const void* sW, void* out,
