@@ -700,6 +700,14 @@ size_t snx_w4a16_batch_cost(size_t M, size_t N, size_t K) {
     return 20 + meet + (units + ncu - 1) / ncu * (25 + steps * step);
 }
 
+// Whether whole-K workgroups are more than a round of the CUs and leave more than
+// a sixth of their rounds idle.
+int snx_w4a16_batch_uneven(size_t M, size_t N) {
+    const size_t rows = (size_t)rows_of((int)M), ncu = (size_t)snx::cu_count();
+    const size_t units = ((N + BN - 1) / BN) * ((M + rows - 1) / rows);
+    return units > ncu && 6 * units < 5 * ncu * ((units + ncu - 1) / ncu);
+}
+
 size_t snx_w4a16_batch_part_bytes(size_t M, size_t N, int splits) {
     const size_t rows = (size_t)rows_of((int)M), tiles = ((N + BN - 1) / BN) * ((M + rows - 1) / rows);
     return tiles * (size_t)splits * rows * BN * sizeof(float);

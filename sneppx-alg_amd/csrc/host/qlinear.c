@@ -226,6 +226,41 @@ static int w4_short(size_t M, size_t N, size_t K, int group, int glu) {
     return (K >= 8192 && N <= 1536) || (!glu && K >= 7168 && K <= 8192 && N >= 1024 && N <= 2048);
 }
 
+/* 2 to 16 rows of so many columns that much of the batch kernel's last round of the
+ * CUs stays idle: split-K, or the small kernels (M = 8, K = 5120: N = 36864 36 / 52
+ * us, 49152 45 / 54, 65536 58 / 56; stacked gate/up rows of K = 8192, F = 20480 69 /
+ * 80, 28672 93 / 83). */
+static int w4_uneven(size_t M, size_t N, size_t K, int group) {
+    return M <= 16 && (snx_w4a16_splitk_span(M, K, group) >= 512 || snx_w4a16_small_ok(M, K, group, 0)) &&
+           snx_w4a16_batch_uneven(M, N);
+}
+
+/* SwiGLU blocks whose projection runs the persistent kernel or the small one, in
+ * fp32 rows and the rule's own pass, where those two launches take less than the
+ * batch kernel's one (us of both / the batch kernel).
+ * Persistent kernel, 9 to 16 rows (up to 8 always: 20.8 / 22.5 at F = 14336):
+ *   K = 1024: F = 256 6.0 / 6.5, 5504 6.4 / 7.3, 6144 6.6 / 7.4, 6656 7.7 / 7.5
+ *   K = 2048: F = 4096 9.1 / 8.5 (M = 9 8.2 / 8.4), 5504 9.0 / 10.1, 6144 9.3 / 10.2,
+ *             6656 11.0 / 10.2, 16384 17.4 / 12.4, 20480 20.4 / 21.6, 24576 23.6 / 21.8
+ *   K = 3072: F = 5504 9.6 / 12.5, 12288 15.6 / 16.2, 13312 17.4 / 16.4, 17408 21 / 29,
+ *             28672 31 / 35
+ *   K = 4096: F = 5504 10.7 / 14.5, 14336 19.9 / 21.4, 14848 21.6 / 21.6, 18432 24 / 41,
+ *             28672 36 / 44
+ * (past F = 16384 the batch kernel's workgroups are more than a round of the CUs).
+ * Small kernel at up to 1024 items of 8 activations: M = 2: K = 1536, F = 1792 6.0 /
+ * 7.5, 3584 7.2 / 7.6, 5504 8.8 / 8.6; K = 2560, F = 5504 10.4 / 11.2, 11008 14.6 /
+ * 13.5; K = 3584, F = 11008 16.1 / 17.3, 14336 17.8 / 17.7; M = 4: K = 2560, F = 2560
+ * 9.8 / 8.3. */
+static int w4_glu_rows(size_t M, size_t F, size_t K, int group) {
+    if (M == 1) return 0;
+    if (snx_w4a16_mt_ok(M, K, group, 0))
+        return M <= 8 || (K == 1024   ? F <= 6144
+                          : K == 2048 ? (F > 5120 && F <= 6144) || (F > 16384 && F <= 20480) || (M <= 10 && F <= 1024)
+                          : K == 3072 ? F <= 12288 || F > 16384
+                                      : F <= 14336 || F > 16384);
+    return snx_w4a16_small_ok(M, K, group, 0) && K >= 1536 && M * K <= 8192 && 4 * F <= 13 * K;
+}
+
 /* The scratch that SNEPPX_qlinear_w4a16_noalloc is documented to need:
  * prepared activations from SNX_W4_GEMM_MIN_M rows on, split-K partials for
  * the decode shapes outside the persistent small-M kernel. */
@@ -290,7 +325,7 @@ static int w4a16_linear(const char* who, int noalloc, const uint16_t* x, const u
         return snx_k_w4a16_gemv_mt(x, qweight, scales, qzeros, NULL, y, bias, y_f32, M, N, K, stream);
     }
     if (aligned && !recorded && !w4_small(M, K, group, scales, qzeros) && !w4_short(M, N, K, group, 0) &&
-        snx_w4a16_batch_ok(M, N, K, group, scales, qzeros))
+        !w4_uneven(M, N, K, group) && snx_w4a16_batch_ok(M, N, K, group, scales, qzeros))
         return w4_batch(who, noalloc, x, qweight, scales, qzeros, bias, y, y_f32, M, N, K, group, 0, stream);
     const int kspan = snx_w4a16_splitk_span(M, K, group);
     if (!g_idx && (M > 4 || (M > 1 && !snx_w4a16_small_ok(M, K, group, 0))) && kspan &&
@@ -439,10 +474,8 @@ int SNEPPX_qlinear_w4a16_swiglu(const uint16_t* x, const uint32_t* qweight,
                                               group, Mp, stream);
         return rc;
     }
-    /* (up to 8 rows of the persistent decode kernel's shapes its fp32 rows and
-     * the rule's own pass stay faster: 20.8 against 22.5 us at F = 14336) */
-    if (aligned && !recorded && !(M <= 8 && snx_w4a16_mt_ok(M, K, group, 0)) && !(M == 1 && w4_small(M, K, group, scales, qzeros)) &&
-        !w4_short(M, 2 * F, K, group, 1) &&
+    if (aligned && !recorded && !w4_glu_rows(M, F, K, group) && !(M == 1 && w4_small(M, K, group, scales, qzeros)) &&
+        !w4_short(M, 2 * F, K, group, 1) && !w4_uneven(M, 2 * F, K, group) &&
         snx_w4a16_batch_ok(M, 2 * F, K, group, scales, qzeros))
         return w4_batch("qlinear_w4a16_swiglu", 0, x, qweight, scales, qzeros, bias, out, 0, M, F, K, group, 1, stream);
     /* other shapes: the [M][2F] projection in fp32 scratch, then the same rule */

@@ -216,6 +216,7 @@ int snx_w4a16_gemv_supported(size_t M, size_t N, size_t K, int group);
 int snx_w4a16_batch_ok(size_t M, size_t N, size_t K, int group, const void* scales, const void* qzeros);
 int snx_w4a16_batch_splits(size_t M, size_t N, size_t K);
 size_t snx_w4a16_batch_cost(size_t M, size_t N, size_t K);
+int snx_w4a16_batch_uneven(size_t M, size_t N);
 size_t snx_w4a16_batch_part_bytes(size_t M, size_t N, int splits);
 size_t snx_w4a16_batch_cnt_bytes(size_t M, size_t N);
 int snx_k_w4a16_batch(const uint16_t* x, const uint32_t* qw, const uint16_t* scales, const uint32_t* qzeros,

@@ -113,3 +113,30 @@ def test_recorded_call_with_a_workspace(lib, make, shape, larger, warmed):
     eager(call2, y2, want2)
     lib.fn["SNEPPX_qlinear_release_workspaces"](st)
     s.synchronize()
+
+
+def test_torch_graph_takes_its_workspaces_apart(lib):
+    """The same under torch.cuda.graph, whose capture refuses allocations of every
+    thread that has not relaxed its own mode, on a stream that has run nothing."""
+    print("[gpu] torch graph: split-K, SwiGLU block, GEMM in spans", flush=True)
+    s = torch.cuda.Stream()
+    made = [_linear(lib, 16, 2048, 14336), _mlp(lib, 32, 1024, 2048), _linear(lib, 512, 1024, 4096)]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        for _, _, call in made:
+            call(s.cuda_stream)
+    for rep in range(3):
+        with torch.cuda.stream(s):
+            for y, _, _ in made:
+                y.fill_(float("nan"))
+            if rep == 1:
+                for _, _, call in made:
+                    call(s.cuda_stream)         # eagerly, in the same workspaces
+            graph.replay()
+        s.synchronize()
+        for y, want, _ in made:
+            assert float((y.double() - want).norm() / want.norm()) <= 4e-3
+    del graph
+    lib.fn["SNEPPX_qlinear_release_workspaces"](s.cuda_stream)
+    s.synchronize()

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from test_gpu_qlinear import DEV, bf16_bits, bf16_to_f32, to_dev
-from test_gpu_w4_batch import _case
+from test_gpu_w4_batch import _case, test_w4_batch_swiglu_matches_float64 as swiglu_matches_float64
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +34,16 @@ def test_both_sides_of_the_short_lines(lib, oracle, M, N, K):
         assert (np.abs(y.cpu().numpy() - want) <= bound).all()
         ys.append(y)
     assert torch.equal(*ys)
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 33000, 640), (16, 32768, 640), (17, 33000, 640)])
+def test_more_columns_than_a_round_of_the_cus(lib, oracle, M, N, K):
+    test_both_sides_of_the_short_lines(lib, oracle, M, N, K)
+
+
+@pytest.mark.parametrize("M,F,K", [
+    (9, 6144, 1024), (9, 6152, 1024), (16, 5128, 2048), (16, 5120, 2048), (12, 12296, 3072), (12, 12288, 3072),
+    (16, 16392, 1024), (2, 4992, 1536), (2, 5000, 1536), (3, 4000, 2560), (4, 4000, 2560), (9, 16392, 640),
+])
+def test_both_sides_of_the_swiglu_lines(lib, oracle, M, F, K):
+    swiglu_matches_float64(lib, oracle, M, F, K, 128, True, False)
