@@ -385,17 +385,33 @@ size_t tiles_of(size_t M, size_t N, size_t rows) { return ((N + BN - 1) / BN) * 
 // with 32 rows 25.2 us).
 size_t rows_of(size_t M, size_t N) { return tiles_of(M, N, 32) * 4 <= (size_t)snx::cu_count() ? 32 : 64; }
 
+// Where the three-piece form is the faster one (us of the GEMV / of it).
+// K % 16 == 0: M = 5: K = 256, N = 256 11.2 / 6.8, K = 1024, N = 4096 10.8 / 10.9;
+// M = 4: K = 1024, N = 4096 9.1 / 11, K = 2048, N = 4096 13.8 / 12.0, 12288 17.6 / 19.2,
+// 24576 33 / 26; M = 3: K = 2048, N = 4096 11.1 / 12, K = 3072, N = 4096 14.3 / 13.2, 12288
+// 23.2 / 24.6, 36864 (just past a round of the CUs) 61 / 73; M = 2: K = 4096, N = 2048
+// 12.3 / 12.9, 4096 14.4 / 13.9, 12288 22 / 29, K = 6144, N = 512 13.3 / 13.2, K = 8192, N =
+// 4096 24.5 / 17.0, 12288 44 / 50.
+// Other K, where the GEMV loads single values: M = 5, N = 4096: K = 260 6.1 / 7.6, 772
+// 10.4 / 10.7, 1000 12.8 / 11.0, N = 16384, K = 20 8.1 / 7.0; N = 256, K = 20: M = 12 5.8 / 6.8,
+// 16 7.2 / 6.6; M = 2, K = 4100, N = 300 15.9 / 11.5.
+bool rows_pay(size_t M, size_t N, size_t K) {
+    if (K % 16 != 0) return M >= 5 ? N > 8192 || M * (K + 600) >= 7500 : M >= 2 && M * K >= 8192;
+    if (M == 2) return N <= 8192 && K >= (N >= 4096 ? 4096u : 6144u);
+    if (M == 3) return K >= (N > 8192 ? 4096u : 2816u) && (N <= 32768 || N > 40960);
+    if (M == 4) return K >= (N > 8192 && N < 16384 ? 3072u : 2048u);
+    return M >= 5;
+}
+
 }  // namespace
 
 extern "C" {
 
 // K a multiple of 4 (rows of weights on their 4-byte alignment), 31-bit buffer
-// offsets.  The rows from which the three-piece form is the faster one: M = 2
-// at K = 4096 (15.0 against 16.1 us at N = 4096), 4 at 2048 (12.6 against
-// 14.4; 3 rows 12.6 against 11.7), 5 at 1024 and less (10.7 against 10.8).
+// offsets, and rows_pay().
 int snx_w8_batch_ok(size_t M, size_t N, size_t K, const void* q) {
     const size_t steps = (K + BK - 1) / BK;
-    return (M >= 5 || (M >= 2 && M * K >= 8192)) && K % 4 == 0 && ((uintptr_t)q & 3u) == 0 && N * K < (1ull << 31) &&
+    return rows_pay(M, N, K) && K % 4 == 0 && ((uintptr_t)q & 3u) == 0 && N * K < (1ull << 31) &&
            M * steps * XSTEP < (1ull << 31) && (M + 64) * N * 4 < (1ull << 31) && M <= 32 * 65535ull;
 }
 

@@ -156,7 +156,7 @@ int snx_k_w4_gptq_quantize(const float* w, const int32_t* g_idx, size_t G, uint3
 /* bias (fp32 [N] or NULL) is added to the fp32 result of every linear below */
 int snx_k_w8_gemv(const float* x, const int8_t* q, const float* s, float* y, const float* bias,
                   size_t M, size_t N, size_t K, void* stream);
-/* the same for M >= 2 on the matrix cores (w8_batch_kernels.hip): x in three
+/* the same for several rows on the matrix cores (w8_batch_kernels.hip): x in three
  * bf16 pieces (xp), K in `splits` spans (partials, and counters that are zero
  * when taken and left zero, with splits > 1) */
 int snx_w8_batch_ok(size_t M, size_t N, size_t K, const void* q);

@@ -25,9 +25,9 @@ def _run(lib, x, q, s, b=None):
 
 
 @pytest.mark.parametrize("M,N,K,bias,mean", [
-    (2, 300, 4096, False, 0.0),     # the fewest rows that take it
+    (2, 300, 6144, False, 0.0),     # the fewest rows that take it
     (5, 1, 64, False, 0.0),         # one column, one step
-    (5, 130, 20, True, 0.0),        # less than a step, 4-byte aligned rows
+    (13, 130, 20, True, 0.0),       # less than a step, 4-byte aligned rows
     (7, 129, 4036, False, 1.0),     # 4036 = 63 steps and 4 columns
     (31, 128, 1040, True, 0.0),
     (32, 257, 8192, False, 0.0),    # many spans
@@ -93,3 +93,11 @@ def test_w8_batch_tiny_activations(lib, size):
     want = x.astype(np.float64) @ q.astype(np.float64).T
     y = _run(lib, x, q, np.ones(300, np.float32))
     assert np.abs(y - want).max() <= 2e-6 * np.abs(want).max() + 2.0**-149
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (2, 300, 4096), (2, 4096, 4096), (2, 8193, 6144), (3, 8193, 3072), (3, 8192, 2816), (4, 9000, 2048), (4, 300, 2048),
+    (5, 300, 260), (5, 8193, 20), (12, 200, 20), (5, 100, 1000),
+])
+def test_both_sides_of_the_rows_line(lib, M, N, K):
+    test_w8_batch_matches_float64(lib, M, N, K, True, 0.0)
