@@ -72,6 +72,17 @@ __device__ __forceinline__ uint32_t e8m0x4(uint32_t s) {
     return u - nz;
 }
 
+// The kernel's arguments, as one: the runtime takes about 20 ns for each of a launch
+// (3.8 us for this kernel's fourteen, 3.4 so).
+struct Args {
+    const uint8_t *A, *W;
+    const void *sA, *sW;
+    void* out;
+    const float* bias;
+    int y_f32, M, N, K, per, extra;
+    uint32_t *part, *cnt;
+};
+
 template <int KIND, int MT>
 struct layout {
     static constexpr int A = 32 * MT * ROWB, W = BN * ROWB;
@@ -87,9 +98,14 @@ struct layout {
 // K % 128 != 0 (int8, fp8): pieces past K are loaded as zeros.
 template <int KIND, int MT, int RING>
 __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(KW, KW))) k_q8_batch(
-    const uint8_t* __restrict__ A, const void* __restrict__ sA, const uint8_t* __restrict__ W,
-    const void* __restrict__ sW, void* __restrict__ out, const float* __restrict__ bias, int y_f32, int M, int N,
-    int K, int per, int extra, uint32_t* __restrict__ part, uint32_t* __restrict__ cnt) {
+    const Args p) {
+    const uint8_t* __restrict__ const A = p.A;
+    const uint8_t* __restrict__ const W = p.W;
+    const void *__restrict__ const sA = p.sA, *__restrict__ const sW = p.sW;
+    void* __restrict__ const out = p.out;
+    const float* __restrict__ const bias = p.bias;
+    const int y_f32 = p.y_f32, M = p.M, N = p.N, K = p.K, per = p.per, extra = p.extra;
+    uint32_t *__restrict__ const part = p.part, *__restrict__ const cnt = p.cnt;
     typedef layout<KIND, MT> L;
     typedef std::conditional_t<KIND == INT8, i32x16, f32x16> acc_t;
     constexpr int STEP = kind_step(KIND), PB = kind_piece(KIND);
@@ -399,8 +415,8 @@ int launch(const Batch& a) {
                                           &part, &cnt))
         return -1;
     const dim3 grid((a.N + BN - 1) / BN, splits, (a.M + 32 * MT - 1) / (32 * MT));
-    k_q8_batch<KIND, MT, RING><<<grid, 256 * KW, bytes, a.s>>>(a.A, a.sA, a.W, a.sW, a.out, a.bias, a.y_f32, a.M, a.N,
-                                                             a.K, steps / splits, steps % splits, static_cast<uint32_t*>(part), cnt);
+    k_q8_batch<KIND, MT, RING><<<grid, 256 * KW, bytes, a.s>>>(Args{a.A, a.W, a.sA, a.sW, a.out, a.bias, a.y_f32, a.M, a.N, a.K,
+        steps / splits, steps % splits, static_cast<uint32_t*>(part), cnt});
     return snx_launch_check("k_q8_batch");
 }
 

@@ -94,6 +94,19 @@ constexpr int OFF_S = BN * BK / 2, OFF_Z = OFF_S + 4 * 256, LDS_B = OFF_Z + 4 * 
 constexpr int lds_stage(int rows) { return lds_a(rows) + LDS_B; }
 constexpr int lds_bytes(int rows, int ring) { return KW * ring * lds_stage(rows); }
 
+// (one argument: see k_q8_batch)
+struct Args {
+    const uint16_t* x;
+    const uint32_t* qw;
+    const uint16_t* scales;
+    const uint32_t* qz;
+    void* y;
+    const float* bias;
+    int y_f32, M, N, K, gshift, glu, per, extra;
+    float* part;
+    uint32_t* cnt;
+};
+
 // One workgroup: 4 KW waves.  Wave (nw, kw) computes output columns
 // n0 + 32 nw .. + 31 for all MT * MR activation rows of the block over wave
 // group kw's share of the workgroup's steps.  MR is the row count of the
@@ -116,9 +129,14 @@ constexpr int lds_bytes(int rows, int ring) { return KW * ring * lds_stage(rows)
 // span order by the last wave to arrive; no wave waits for another.
 template <int MR, int MT, int GS, int RING>
 __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(KW, KW))) k_w4a16_batch(
-    const uint16_t* __restrict__ x, const uint32_t* __restrict__ qw, const uint16_t* __restrict__ scales,
-    const uint32_t* __restrict__ qz, void* __restrict__ y, const float* __restrict__ bias, int y_f32, int M,
-    int N, int K, int gshift, int glu, int per, int extra, float* __restrict__ part, uint32_t* __restrict__ cnt) {
+    const Args p) {
+    const uint16_t *__restrict__ const x = p.x, *__restrict__ const scales = p.scales;
+    const uint32_t *__restrict__ const qw = p.qw, *__restrict__ const qz = p.qz;
+    void* __restrict__ const y = p.y;
+    const float* __restrict__ const bias = p.bias;
+    const int y_f32 = p.y_f32, M = p.M, N = p.N, K = p.K, gshift = p.gshift, glu = p.glu, per = p.per, extra = p.extra;
+    float* __restrict__ const part = p.part;
+    uint32_t* __restrict__ const cnt = p.cnt;
     typedef mfma_of<MR> MF;
     typedef typename MF::acc_t acc_t;
     constexpr int ROWS = MT * MR, NS = 32 / MR, LQ = 64 / MR;   // NS column subtiles, LQ lane groups along k
@@ -632,8 +650,8 @@ int launch(const Batch& a) {
     const dim3 grid((a.N + cols - 1) / cols, a.splits, (a.M + MT * MR - 1) / (MT * MR));
     const int steps = a.K / BK;
     k_w4a16_batch<MR, MT, GS, RING><<<grid, 256 * KW, bytes, a.s>>>(
-        a.x, a.qw, a.scales, a.qz, a.y, a.bias, a.y_f32, a.M, a.N, a.K, a.gshift, a.glu, steps / a.splits, steps % a.splits,
-        a.part, a.cnt);
+        Args{a.x, a.qw, a.scales, a.qz, a.y, a.bias, a.y_f32, a.M, a.N, a.K, a.gshift, a.glu, steps / a.splits,
+             steps % a.splits, a.part, a.cnt});
     return snx_launch_check("k_w4a16_batch");
 }
 

@@ -93,6 +93,17 @@ struct layout {
     static constexpr int PLANE = 32 * MT * 128, A = 3 * PLANE, W = BN * 64, STAGE = A + W;
 };
 
+// (one argument: see k_q8_batch)
+struct Args {
+    const uint16_t* xp;
+    const int8_t* qw;
+    const float *scales, *bias;
+    float* y;
+    int M, N, K, per, extra;
+    float* part;
+    uint32_t* cnt;
+};
+
 // four int8 of a word as two registers of bf16 pairs (exact)
 __device__ __forceinline__ void bytes_to_bf16(uint32_t w, uint32_t& lo, uint32_t& hi) {
     const float f0 = (float)(int8_t)w, f1 = (float)(int8_t)(w >> 8);
@@ -111,9 +122,13 @@ __device__ __forceinline__ void bytes_to_bf16(uint32_t w, uint32_t& lo, uint32_t
 // comments cover what is not said here.
 template <int MT, int KW, int RING>
 __global__ void __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(KW, KW))) k_w8_batch(
-    const uint16_t* __restrict__ xp, const int8_t* __restrict__ qw, const float* __restrict__ scales,
-    const float* __restrict__ bias, float* __restrict__ y, int M, int N, int K, int per, int extra,
-    float* __restrict__ part, uint32_t* __restrict__ cnt) {
+    const Args p) {
+    const uint16_t* __restrict__ const xp = p.xp;
+    const int8_t* __restrict__ const qw = p.qw;
+    const float *__restrict__ const scales = p.scales, *__restrict__ const bias = p.bias;
+    float *__restrict__ const y = p.y, *__restrict__ const part = p.part;
+    uint32_t* __restrict__ const cnt = p.cnt;
+    const int M = p.M, N = p.N, K = p.K, per = p.per, extra = p.extra;
     typedef layout<MT> L;
     constexpr int AL = 3 * MT, WL = 2, PER = AL + WL;
     constexpr int NP = 4 * MT, OWN = NP / KW;     // 16-byte result pieces per lane, and those a wave finishes
@@ -371,8 +386,8 @@ int launch(const Batch& a) {
     }
     const dim3 grid((a.N + BN - 1) / BN, a.splits, (a.M + 32 * MT - 1) / (32 * MT));
     const int steps = (a.K + BK - 1) / BK;
-    k_w8_batch<MT, KW, RING><<<grid, 256 * KW, bytes, a.s>>>(a.xp, a.qw, a.scales, a.bias, a.y, a.M, a.N, a.K,
-                                                           steps / a.splits, steps % a.splits, a.part, a.cnt);
+    k_w8_batch<MT, KW, RING><<<grid, 256 * KW, bytes, a.s>>>(
+        Args{a.xp, a.qw, a.scales, a.bias, a.y, a.M, a.N, a.K, steps / a.splits, steps % a.splits, a.part, a.cnt});
     return snx_launch_check("k_w8_batch");
 }
 
