@@ -9,17 +9,18 @@
 // the chip is full, so the kernel is about filling it: 128 output columns per
 // workgroup leave 14 to 224 workgroups for a whole K, and K is split, first
 // over the wave groups of a workgroup (their sums meet in LDS), then over
-// workgroups (their sums meet in memory, about 2.5 us).  A step then costs
-// its instructions: 1300 cycles of two waves per SIMD at 16 rows without any
-// load, 1800 with them, half of it the nibble unpack; and a launch its code,
-// 0.6 us per KB read once from a cold instruction cache.
-// Measured (graph replay, weights from HBM, before: 64-row slices of
-// k_w4a16_gemv, k_w4a16_splitk and, with groups of 32 and 64,
+// workgroups (their sums meet in memory, about 2.5 us).  What is left is
+// latency more than any unit: the vector units are busy for 27 % of the
+// cycles and the matrix cores for 10 at 16 rows (N = 4096, K = 14336), 26 and
+// 36 at 96 (N = 6144, K = 4096); and a launch reads its code, 0.6 us per KB
+// from a cold instruction cache.
+// Measured (calls in a loop over eight sets of weights, before: 64-row slices
+// of k_w4a16_gemv, k_w4a16_splitk and, with groups of 32 and 64,
 // k_w4a16_generic):
-//   N = 6144,  K = 4096:  M = 32 22.0 -> 11.1 us, 96 57.7 -> 18.8, 192 107 -> 26
-//   N = 28672, K = 4096:  M = 32 80 -> 26 us, 96 193 -> 43
-//   N = 4096,  K = 14336: M = 16 21.2 -> 18.1 us, 96 179 -> 31
-//   N = 6144,  K = 4096, groups of 64: M = 16 460 -> 10.7 us
+//   N = 6144,  K = 4096:  M = 32 21.7 -> 10.9 us, 96 57.3 -> 18.0, 192 107 -> 25.5
+//   N = 28672, K = 4096:  M = 32 79 -> 24.3 us, 96 195 -> 46
+//   N = 4096,  K = 14336: M = 16 19.7 -> 16.6 us, 96 176 -> 30.3
+//   N = 6144,  K = 4096, groups of 64: M = 16 459 -> 10.6 us, 96 2714 -> 18.5
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

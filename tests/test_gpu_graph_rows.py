@@ -1,6 +1,6 @@
 """Linears with several rows recorded into a graph on a stream that has not run
 them: the recorded call takes no workspace (which other calls and replays would
-share, and a larger call replace), before and after an eager call on the same
+share), before and after an eager call on the same
 stream, and every replay gives the float64 product."""
 import numpy as np
 import pytest
