@@ -231,7 +231,8 @@ static int w4_short(size_t M, size_t N, size_t K, int group, int glu) {
  * us, 49152 45 / 54, 65536 58 / 56; stacked gate/up rows of K = 8192, F = 20480 69 /
  * 80, 28672 93 / 83). */
 static int w4_uneven(size_t M, size_t N, size_t K, int group) {
-    return M <= 16 && (snx_w4a16_splitk_span(M, K, group) >= 512 || snx_w4a16_small_ok(M, K, group, 0)) &&
+    return M >= 2 && M <= 16 &&
+           (snx_w4a16_splitk_span(M, K, group) >= 512 || snx_w4a16_small_ok(M, K, group, 0)) &&
            snx_w4a16_batch_uneven(M, N);
 }
 

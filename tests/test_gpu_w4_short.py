@@ -36,7 +36,7 @@ def test_both_sides_of_the_short_lines(lib, oracle, M, N, K):
     assert torch.equal(*ys)
 
 
-@pytest.mark.parametrize("M,N,K", [(8, 33000, 640), (16, 32768, 640), (17, 33000, 640)])
+@pytest.mark.parametrize("M,N,K", [(8, 33000, 640), (16, 32768, 640), (17, 33000, 640), (1, 33000, 640)])
 def test_more_columns_than_a_round_of_the_cus(lib, oracle, M, N, K):
     test_both_sides_of_the_short_lines(lib, oracle, M, N, K)
 
