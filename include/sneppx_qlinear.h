@@ -105,7 +105,8 @@ int SNEPPX_dev_quantize_fp8_e4m3_scaled(const float* in, uint8_t* out, float* sc
 /* ---- quantized linears ---------------------------------------------------- */
 
 /* C1: W8 weight-only, fp32 activations: y[m][n] = s[n] * sum_k x[m][k]*q[n][k]
- * (+ bias[n]) in fp32.  x fp32 [M][K], y fp32 [M][N].  Decode GEMV, HBM-bound. */
+ * (+ bias[n]) in fp32.  x fp32 [M][K], y fp32 [M][N].  Decode GEMV, HBM-bound;
+ * several rows on the matrix cores, x cut exactly into bf16 pieces. */
 int SNEPPX_qlinear_w8_gemv(const float* x, const int8_t* qweight, const float* scales,
                            const float* bias, float* y, size_t M, size_t N, size_t K,
                            SNEPPXStream stream);
